@@ -22,16 +22,14 @@ namespace {
 constexpr int kTile = 64;
 constexpr float kGeluC = 0.7978845608028654f;
 
-__device__ __forceinline__ float gelu_f(float x) {
-  const float u = kGeluC * (x + 0.044715f * x * x * x);
-  return 0.5f * x * (1.0f + tanhf(u));
-}
-
-__device__ __forceinline__ float gelu_grad(float x) {
-  const float u = kGeluC * (x + 0.044715f * x * x * x);
-  const float th = tanhf(u);
+// th = gelu_tanh(x) serves both gelu(x) and its derivative
+__device__ __forceinline__ float gelu_tanh(float x) { return tanhf(kGeluC * (x + 0.044715f * x * x * x)); }
+__device__ __forceinline__ float gelu_f(float x, float th) { return 0.5f * x * (1.0f + th); }
+__device__ __forceinline__ float gelu_grad(float x, float th) {
   return 0.5f * (1.0f + th) + 0.5f * x * (1.0f - th * th) * kGeluC * (1.0f + 3.0f * 0.044715f * x * x);
 }
+__device__ __forceinline__ float gelu_f(float x) { return gelu_f(x, gelu_tanh(x)); }
+__device__ __forceinline__ float gelu_grad(float x) { return gelu_grad(x, gelu_tanh(x)); }
 
 template <typename T>
 __device__ __forceinline__ float ld(const T* p, size_t i);
@@ -40,6 +38,15 @@ __device__ __forceinline__ float ld<float>(const float* p, size_t i) { return p[
 template <>
 __device__ __forceinline__ float ld<__hip_bfloat16>(const __hip_bfloat16* p, size_t i) {
   return __bfloat162float(p[i]);
+}
+
+// Barrier of a workgroup whose waves exchange data through LDS only: waits
+// for LDS traffic, not for global loads and stores in flight (__syncthreads
+// waits for those too, which ends every prefetch at each barrier).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // bf16 operands for the matrix cores: round to nearest even, as
@@ -466,22 +473,12 @@ __global__ void sum_splits(const float* part, int n, int splits, float* out) {
   out[e] = s;
 }
 
-__device__ __forceinline__ void adam_update(int i, float gi, float* p, float* m, float* v, __hip_bfloat16* w16,
-                                            float lr, float b1, float b2, float eps, float bc1, float bc2) {
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float pi = p[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
-  p[i] = pi;
-  if (w16) w16[i] = __float2bfloat16(pi);
-}
-
-__global__ void adam_step(float* p, const float* g, float* m, float* v, __hip_bfloat16* w16, int n,
-                          float lr, float b1, float b2, float eps, float bc1, float bc2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  adam_update(i, g[i], p, m, v, w16, lr, b1, b2, eps, bc1, bc2);
+// One parameter p with moments m, v and gradient g.
+__device__ __forceinline__ void adam_update(float g, float& p, float& m, float& v, float lr, float b1, float b2,
+                                            float eps, float bc1, float bc2) {
+  m = b1 * m + (1.f - b1) * g;
+  v = b2 * v + (1.f - b2) * g * g;
+  p = p - lr * (m / bc1) / (sqrtf(v / bc2) + eps);
 }
 
 // Adam with each gradient summed from its split-K partials, part[k stride +
@@ -494,7 +491,12 @@ __global__ void adam_step_splits(float* p, const float* part, int splits, size_t
   if (i >= n) return;
   float g = 0.f;
   for (int k = 0; k < splits; ++k) g += part[k * stride + i];
-  adam_update(i, g, p, m, v, w16, lr, b1, b2, eps, bc1, bc2);
+  float pi = p[i], mi = m[i], vi = v[i];
+  adam_update(g, pi, mi, vi, lr, b1, b2, eps, bc1, bc2);
+  p[i] = pi;
+  m[i] = mi;
+  v[i] = vi;
+  w16[i] = __float2bfloat16(pi);
 }
 
 __global__ void to_bf16(const float* src, __hip_bfloat16* dst, int n) {

@@ -9,11 +9,15 @@
 // Loss = mean over the batch of 0.5 (A_L - target)^2.  Adam follows Kingma
 // & Ba (2015), Algorithm 1 (bias-corrected moments).
 //
-// GEMMs: 64x64 output tiles, 256 threads (four waves of 2x2 16x16 MFMA
-// blocks), K in steps of 32 staged through LDS as bf16.  Weight gradients
-// reduce over the batch in row splits whose partials are summed in order;
-// bias gradients (column sums of the fp32 gradients) likewise, so every
-// reduction has a fixed order and training is deterministic.
+// Networks of up to kDenseMaxLayers layers of at most kDenseMaxWidth units
+// (the surrogate is 64-256-256-1) run as the fused kernels of mh_dense.h:
+// one launch forward, two per training step.  Wider ones run a launch per
+// layer and direction: 64x64 output tiles, 256 threads (four waves of 2x2
+// 16x16 MFMA blocks), K in steps of 32 staged through LDS as bf16.  Weight
+// gradients reduce over the batch in row splits whose partials are summed in
+// order; bias gradients (column sums of the fp32 gradients) likewise, so
+// every reduction has a fixed order and training is deterministic, with the
+// same bits on both paths.
 #include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
 
@@ -27,7 +31,7 @@
 
 #include "mercury_hip.h"
 #include "mh_internal.h"
-#include "mh_nn_kernels.h"
+#include "mh_dense.h"
 
 // Scratch of mh_mlp_forward_noalloc: the hidden activations of one call, in
 // two halves that alternate between layers.  Every device holds its own
@@ -43,7 +47,12 @@ struct mh_mlp {
   std::vector<size_t> w_off;  // offset of W_l in the parameter vector; b_l follows W_l
   size_t n_params = 0;
   Dev<float> params, grads, m, v;
-  Dev<__hip_bfloat16> w16;    // bf16 copy of the whole parameter vector (weights used)
+  bool fused = false;         // every layer fits the fused kernels
+  DenseShape shape{};         // fused: the layers and where their packed weights lie
+  Dev<uint16_t> pack;         // fused: bf16 weights in the kernels' operand order
+  std::vector<Dev<uint16_t>> X16, D16;  // fused: weight-gradient operands of a batch
+  std::vector<Dev<float>> delta;        // fused: gradients of every layer's output
+  Dev<__hip_bfloat16> w16;    // otherwise: bf16 copy of the whole parameter vector (weights used)
   std::vector<Dev<float>> Z, A, dA;  // per layer activations / gradients
   Dev<float> x, t, dY, terms, data_x, data_t;
   Dev<float> epoch_terms;     // loss terms of every batch of a training run's last epoch
@@ -65,9 +74,30 @@ namespace {
 // splits (at least 64 rows each), summed in order
 constexpr int kMlpSplit = 8;
 
+// Row splits of a batch of B for the weight and bias gradients.
+int mlp_splits(int B) { return std::max(1, std::min(kMlpSplit, B / 64)); }
+
 void ensure_batch(mh_mlp* net, int B) {
   if (B <= net->batch_cap) return;
   const int L = net->L();
+  if (net->fused) {
+    // operands are padded to whole slices of 32 rows per split: their size
+    // is not monotonic in B, so a bound for every smaller batch is kept
+    const size_t rows = static_cast<size_t>(B) + 32 * kMlpSplit;
+    net->X16.resize(L);
+    net->D16.resize(L);
+    net->delta.resize(L);
+    for (int l = 0; l < L; l++) {
+      net->X16[l].ensure(rows * ((net->sizes[l] + 15) / 16 * 16));
+      net->D16[l].ensure(rows * ((net->sizes[l + 1] + 15) / 16 * 16));
+      net->delta[l].ensure(static_cast<size_t>(B) * net->sizes[l + 1]);
+    }
+    net->x.ensure(static_cast<size_t>(B) * net->sizes[0]);
+    net->t.ensure(static_cast<size_t>(B) * net->sizes[L]);
+    net->terms.ensure(static_cast<size_t>(B) * net->sizes[L]);
+    net->batch_cap = B;
+    return;
+  }
   net->Z.resize(L);
   net->A.resize(L);
   net->dA.resize(L + 1);
@@ -81,6 +111,56 @@ void ensure_batch(mh_mlp* net, int B) {
   net->dY.ensure(static_cast<size_t>(B) * net->sizes[L]);
   net->terms.ensure(static_cast<size_t>(B) * net->sizes[L]);
   net->batch_cap = B;
+}
+
+// Brings the device weights (packed, or the bf16 copy) up to date with the
+// fp32 parameters.
+void refresh_weights(mh_mlp* net) {
+  if (net->fused) {
+    for (int l = 0; l < net->L(); l++) {
+      const PackedLayer& p = net->shape.layer[l];
+      hipLaunchKernelGGL(pack_layer, dim3((p.out * p.in + 255) / 256), dim3(256), 0, net->stream, p, net->params.p,
+                         net->pack.p);
+    }
+  } else {
+    hipLaunchKernelGGL(to_bf16, dim3((net->n_params + 255) / 256), dim3(256), 0, net->stream, net->params.p,
+                       net->w16.p, static_cast<int>(net->n_params));
+  }
+  hipcheck(hipGetLastError(), "weights");
+}
+
+// Fused forward of B rows on the device, x -> y.  A workgroup reads every
+// packed weight from L2, so large batches take taller row tiles; small ones
+// take 16 rows, as long as one workgroup per CU covers them.  64-256-256-1
+// on MI355X, us with tiles of 16 / 32 / 64 rows: 4096 rows 7.7 / 10.9 / 18.6
+// (the layer-by-layer kernels 13.9), 8192 rows 13.6 / 10.9 / 18.5, 16384
+// rows 25.7 / 20.6 / 18.6, 65536 rows 98 / 78 / 70.
+void fused_forward(mh_mlp* net, const float* x, int B, float* y, hipStream_t s) {
+  if (B <= 4096) launch_dense_net<1, false>(net->shape, net->params.p, net->pack.p, x, B, y, DenseTrain{}, s);
+  else if (B <= 8192) launch_dense_net<2, false>(net->shape, net->params.p, net->pack.p, x, B, y, DenseTrain{}, s);
+  else launch_dense_net<4, false>(net->shape, net->params.p, net->pack.p, x, B, y, DenseTrain{}, s);
+}
+
+// Fused loss terms and gradients of a batch: batch row r is row x_idx[r] of
+// x and t_idx[r] of target (null: r).  Gradients go to net->grads, or with
+// `adam` straight into the parameters.
+void fused_backward(mh_mlp* net, const float* x, const float* target, const int* idx, int B, float* terms,
+                    const AdamArgs* adam) {
+  DenseTrain tr{};
+  tr.rs = row_splits(B, mlp_splits(B));
+  tr.x_idx = idx;
+  tr.t_idx = idx;
+  tr.target = target;
+  tr.inv_b = 1.0f / B;
+  tr.terms = terms;
+  for (int l = 0; l < net->L(); l++) {
+    tr.X[l] = net->X16[l].p;
+    tr.D[l] = net->D16[l].p;
+    tr.delta[l] = net->delta[l].p;
+  }
+  launch_dense_net<1, true>(net->shape, net->params.p, net->pack.p, x, B, nullptr, tr, net->stream);
+  if (adam) launch_dense_wgrad<4, 1, true>(net->shape, tr, *adam, nullptr, net->stream);
+  else launch_dense_wgrad<4, 1, false>(net->shape, tr, AdamArgs{}, net->grads.p, net->stream);
 }
 
 // Forward of a batch already in net->x (or `in`): activations in A[l].
@@ -103,9 +183,6 @@ void forward(mh_mlp* net, const float* in, int B) {
     prev = net->A[l].p;
   }
 }
-
-// Row splits of a batch of B for the weight and bias gradients.
-int mlp_splits(int B) { return std::max(1, std::min(kMlpSplit, B / 64)); }
 
 // Backward from dY (already (Y - T)/B): gradients into net->grads, or with
 // to_adam their split partials into net->part at the parameters' offsets,
@@ -151,11 +228,15 @@ void backward(mh_mlp* net, const float* in, int B, bool to_adam = false) {
 
 float loss_and_grad(mh_mlp* net, const float* in, const float* target, int B) {
   const int L = net->L();
-  forward(net, in, B);
   const int n = B * net->sizes[L];
-  hipLaunchKernelGGL(loss_grad, dim3((n + 255) / 256), dim3(256), 0, net->stream, net->A[L - 1].p, target, n,
-                     1.0f / B, net->dY.p, net->terms.p);
-  backward(net, in, B);
+  if (net->fused) {
+    fused_backward(net, in, target, nullptr, B, net->terms.p, nullptr);
+  } else {
+    forward(net, in, B);
+    hipLaunchKernelGGL(loss_grad, dim3((n + 255) / 256), dim3(256), 0, net->stream, net->A[L - 1].p, target, n,
+                       1.0f / B, net->dY.p, net->terms.p);
+    backward(net, in, B);
+  }
   std::vector<float> terms(n);
   hipcheck(hipMemcpyAsync(terms.data(), net->terms.p, n * sizeof(float), hipMemcpyDeviceToHost, net->stream),
            "D2H");
@@ -207,10 +288,29 @@ int mh_mlp_create(int device, int n_layers, const int* sizes, uint64_t seed, mh_
       off += static_cast<size_t>(sizes[l + 1]) * sizes[l] + sizes[l + 1];
     }
     net->n_params = off;
-    size_t widest = 0;
-    for (int l = 0; l < n_layers; l++) widest = std::max<size_t>(widest, static_cast<size_t>(sizes[l]) * sizes[l + 1]);
-    // split partials of one tensor, or of every parameter for adam_step_splits
-    net->part.ensure(static_cast<size_t>(kMlpSplit) * std::max(widest, net->n_params));
+    net->fused = n_layers <= kDenseMaxLayers && *std::max_element(sizes, sizes + n_layers + 1) <= kDenseMaxWidth;
+    if (net->fused) {
+      int at = 0;
+      net->shape.L = n_layers;
+      for (int l = 0; l < n_layers; l++) {
+        PackedLayer& p = net->shape.layer[l];
+        p.out = sizes[l + 1];
+        p.in = p.c = sizes[l];
+        p.w_off = static_cast<int>(net->w_off[l]);
+        p.b_off = static_cast<int>(net->b_off(l));
+        at = pack_layout(p, at);
+      }
+      net->shape.zero = at;
+      at += 8;
+      net->pack.ensure(at);
+      hipLaunchKernelGGL(fill_zero_u16, dim3((at + 255) / 256), dim3(256), 0, net->stream, net->pack.p, at);
+    } else {
+      size_t widest = 0;
+      for (int l = 0; l < n_layers; l++) widest = std::max<size_t>(widest, static_cast<size_t>(sizes[l]) * sizes[l + 1]);
+      // split partials of one tensor, or of every parameter for adam_step_splits
+      net->part.ensure(static_cast<size_t>(kMlpSplit) * std::max(widest, net->n_params));
+      net->w16.ensure(off);
+    }
     // He-uniform weights (bound sqrt(6 / fan_in)), zero biases
     std::mt19937_64 rng(seed);
     std::vector<float> p(off, 0.f);
@@ -224,13 +324,11 @@ int mh_mlp_create(int device, int n_layers, const int* sizes, uint64_t seed, mh_
     net->grads.ensure(off);
     net->m.ensure(off);
     net->v.ensure(off);
-    net->w16.ensure(off);
     std::vector<float> zeros(off, 0.f);
     hipcheck(hipMemcpy(net->params.p, p.data(), off * sizeof(float), hipMemcpyHostToDevice), "H2D");
     hipcheck(hipMemcpy(net->m.p, zeros.data(), off * sizeof(float), hipMemcpyHostToDevice), "H2D");
     hipcheck(hipMemcpy(net->v.p, zeros.data(), off * sizeof(float), hipMemcpyHostToDevice), "H2D");
-    hipLaunchKernelGGL(to_bf16, dim3((off + 255) / 256), dim3(256), 0, net->stream, net->params.p, net->w16.p,
-                       static_cast<int>(off));
+    refresh_weights(net.get());
     hipcheck(hipStreamSynchronize(net->stream), "init");
     *out = net.release();
     return MH_OK;
@@ -261,8 +359,7 @@ int mh_mlp_set_params(mh_mlp* net, const float* in) {
     if (!net || !in) throw mh::Error(MH_ERR_ARG, "null argument");
     hipcheck(hipSetDevice(net->device), "hipSetDevice");
     hipcheck(hipMemcpy(net->params.p, in, net->n_params * sizeof(float), hipMemcpyHostToDevice), "H2D");
-    hipLaunchKernelGGL(to_bf16, dim3((net->n_params + 255) / 256), dim3(256), 0, net->stream, net->params.p,
-                       net->w16.p, static_cast<int>(net->n_params));
+    refresh_weights(net);
     hipcheck(hipStreamSynchronize(net->stream), "set params");
     net->adam_t = 0;
     std::vector<float> zeros(net->n_params, 0.f);
@@ -281,6 +378,29 @@ int mh_mlp_forward(mh_mlp* net, const float* x, int batch, float* y) {
     hipcheck(hipSetDevice(net->device), "hipSetDevice");
     const int L = net->L();
     const int chunk = 8192;
+    if (net->fused) {
+      // rows go up in pieces, each followed by its kernel, so all but the
+      // last piece's kernel runs while the host stages the next; results
+      // come back in one copy per round
+      const int ni = net->sizes[0], no = net->sizes[L], round = 16 * chunk;
+      net->x.ensure(static_cast<size_t>(std::min(batch, round)) * ni);
+      net->dY.ensure(static_cast<size_t>(std::min(batch, round)) * no);
+      for (int r0 = 0; r0 < batch; r0 += round) {
+        const int rows = std::min(round, batch - r0);
+        for (int b0 = 0; b0 < rows; b0 += chunk) {
+          const int B = std::min(chunk, rows - b0);
+          hipcheck(hipMemcpyAsync(net->x.p + static_cast<size_t>(b0) * ni, x + static_cast<size_t>(r0 + b0) * ni,
+                                  static_cast<size_t>(B) * ni * sizeof(float), hipMemcpyHostToDevice, net->stream),
+                   "H2D");
+          fused_forward(net, net->x.p + static_cast<size_t>(b0) * ni, B, net->dY.p + static_cast<size_t>(b0) * no,
+                        net->stream);
+        }
+        hipcheck(hipMemcpyAsync(y + static_cast<size_t>(r0) * no, net->dY.p, static_cast<size_t>(rows) * no * sizeof(float),
+                                hipMemcpyDeviceToHost, net->stream), "D2H");
+      }
+      hipcheck(hipStreamSynchronize(net->stream), "sync");
+      return MH_OK;
+    }
     ensure_batch(net, std::min(batch, chunk));
     for (int b0 = 0; b0 < batch; b0 += chunk) {
       const int B = std::min(chunk, batch - b0);
@@ -313,6 +433,10 @@ int mh_mlp_forward_noalloc(mh_mlp* net, const float* x, int batch, float* y, voi
                                         std::to_string(half) + " floats)");
     hipcheck(hipSetDevice(net->device), "hipSetDevice");
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : net->stream;
+    if (net->fused) {
+      fused_forward(net, x, batch, y, s);
+      return MH_OK;
+    }
     const float* prev = x;
     for (int l = 0; l < L; l++) {
       const int ni = net->sizes[l], no = net->sizes[l + 1];
@@ -387,23 +511,28 @@ int mh_mlp_train(mh_mlp* net, const float* x, const float* target, int n, int ba
       hipcheck(hipMemcpyAsync(net->idx.p, perm.data(), n * sizeof(int), hipMemcpyHostToDevice, net->stream), "H2D");
       const bool last = ep == n_epochs - 1;
       for (int b0 = 0; b0 + batch <= n; b0 += batch) {
+        float* terms = last ? net->epoch_terms.p + batches * nt : net->terms.p;
+        net->adam_t++;
+        const float bc1 = 1.f - std::pow(b1, static_cast<float>(net->adam_t));
+        const float bc2 = 1.f - std::pow(b2, static_cast<float>(net->adam_t));
+        if (last) batches++;
+        if (net->fused) {
+          const AdamArgs adam{net->params.p, net->m.p, net->v.p, net->pack.p, lr, b1, b2, eps, bc1, bc2};
+          fused_backward(net, net->data_x.p, net->data_t.p, net->idx.p + b0, batch, terms, &adam);
+          continue;
+        }
         hipLaunchKernelGGL(gather_rows, dim3(batch), dim3(64), 0, net->stream, net->data_x.p, net->idx.p + b0,
                            batch, ni, net->x.p);
         hipLaunchKernelGGL(gather_rows, dim3(batch), dim3(64), 0, net->stream, net->data_t.p, net->idx.p + b0,
                            batch, no, net->t.p);
         forward(net, net->x.p, batch);
-        float* terms = last ? net->epoch_terms.p + batches * nt : net->terms.p;
         hipLaunchKernelGGL(loss_grad, dim3((static_cast<int>(nt) + 255) / 256), dim3(256), 0, net->stream,
                            net->A[L - 1].p, net->t.p, static_cast<int>(nt), 1.0f / batch, net->dY.p, terms);
         backward(net, net->x.p, batch, true);
-        net->adam_t++;
-        const float bc1 = 1.f - std::pow(b1, static_cast<float>(net->adam_t));
-        const float bc2 = 1.f - std::pow(b2, static_cast<float>(net->adam_t));
         hipLaunchKernelGGL(adam_step_splits, dim3((net->n_params + 255) / 256), dim3(256), 0, net->stream,
                            net->params.p, net->part.p, mlp_splits(batch), net->n_params, net->m.p, net->v.p,
                            net->w16.p, static_cast<int>(net->n_params), lr, b1, b2, eps, bc1, bc2);
         hipcheck(hipGetLastError(), "train step");
-        if (last) batches++;
       }
     }
     // the last epoch's mean over batches of each batch's summed terms / batch
