@@ -470,12 +470,29 @@ __global__ __launch_bounds__(kWgThreads) void dense_wgrad(DenseShape sh, DenseTr
     const int c = tid & 15, n = 16 * it + c;
     float pmv[3] = {};
     if (tid < 16 && n < p.out) load(p.b_off + n, pmv);
-    for (int u = tid >> 4; u < rs.splits * 16; u += kWgThreads / 16) {
-      const int s = u >> 4, r1 = min(rs.B, (s + 1) * rs.rows);
-      float sum = 0.f;
-      if (n < p.out)
-        for (int r = s * rs.rows + (u & 15); r < r1; r += 16) sum += delta[static_cast<size_t>(r) * p.out + n];
-      acc[u][c] = sum;
+    // U (split, group) sums at a time, their loads in flight together (no
+    // conditions: a row outside its split is read elsewhere and adds +0)
+    constexpr int U = 8;
+    for (int u0 = tid >> 4; u0 < rs.splits * 16; u0 += U * (kWgThreads / 16)) {
+      float sum[U] = {};
+      for (int i = 0; i < rs.rows; i += 16) {
+        float v[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+          const int u = u0 + k * (kWgThreads / 16), r = (u >> 4) * rs.rows + (u & 15) + i;
+          v[k] = delta[static_cast<size_t>(min(r, rs.B - 1)) * p.out + min(n, p.out - 1)];
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+          const int u = u0 + k * (kWgThreads / 16), in_split = (u & 15) + i;
+          sum[k] += in_split < rs.rows && (u >> 4) * rs.rows + in_split < rs.B ? v[k] : 0.f;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const int u = u0 + k * (kWgThreads / 16);
+        if (u < rs.splits * 16) acc[u][c] = sum[k];
+      }
     }
     lds_barrier();
     for (int u = tid; u < rs.splits * 16; u += kWgThreads) {
@@ -501,58 +518,67 @@ __global__ __launch_bounds__(kWgThreads) void dense_wgrad(DenseShape sh, DenseTr
     if (e < 16 * kCols && o < p.out && i < p.in) load(p.w_off + o * p.in + i, pmv[k]);
   }
   const int nti = (p.out + 15) >> 4, ntj = (p.in + 15) >> 4;
+  // The operands of SR splits (one slice each), or of SR slices of one split
+  // at a time, are requested together, without conditions: rows outside the
+  // split were never written, and count as zeros.
+  f32x4_t acc[SR][JT];
 #pragma unroll
-  for (int k = 0; k < SR; ++k) {
-    const int s = wave + 8 * k;
-    f32x4_t acc[JT];
+  for (int k = 0; k < SR; ++k)
 #pragma unroll
-    for (int j = 0; j < JT; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    if (s < rs.splits) {
-      const int nr = min(rs.B - s * rs.rows, rs.rows);
-      // two slices per round: their loads are in flight together
-      for (int sl = 0; 32 * sl < nr; sl += 2) {
-        u16x8_t d[2], xs[2][JT];
+    for (int j = 0; j < JT; ++j) acc[k][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  struct Operands {
+    u16x8_t d, x[JT];
+  };
+  auto request = [&](int s, int sl) {
+    const size_t slice = static_cast<size_t>(min(s, rs.splits - 1)) * rs.slices + min(sl, rs.slices - 1);
+    Operands o;
+    o.d = *reinterpret_cast<const u16x8_t*>(D + (slice * nti + it) * 512 + 8 * lane);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          // rows of the lane's 8 that lie inside the split: the rest were
-          // never written and count as zeros
-          const int valid = nr - 32 * (sl + u) - 8 * (lane >> 4);
-          const size_t slice = static_cast<size_t>(s) * rs.slices + sl + u;
-          d[u] = u16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int j = 0; j < JT; ++j)
+      o.x[j] = *reinterpret_cast<const u16x8_t*>(X + (slice * ntj + min(jg * JT + j, ntj - 1)) * 512 + 8 * lane);
+    return o;
+  };
+  auto products = [&](int s, int sl, Operands& o, f32x4_t (&c)[JT]) {
+    const int nr = s < rs.splits ? min(rs.B - s * rs.rows, rs.rows) - 32 * sl : 0;  // rows of the slice
+    if (nr <= 0) return;
+    if (nr < 32) {
+      const int valid = nr - 8 * (lane >> 4);
 #pragma unroll
-          for (int j = 0; j < JT; ++j) xs[u][j] = u16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-          if (valid > 0) {
-            d[u] = *reinterpret_cast<const u16x8_t*>(D + (slice * nti + it) * 512 + 8 * lane);
+      for (int e = 0; e < 8; ++e) {
+        o.d[e] = e < valid ? o.d[e] : uint16_t(0);
 #pragma unroll
-            for (int j = 0; j < JT; ++j)
-              if (jg * JT + j < ntj)
-                xs[u][j] = *reinterpret_cast<const u16x8_t*>(X + (slice * ntj + jg * JT + j) * 512 + 8 * lane);
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int valid = nr - 32 * (sl + u) - 8 * (lane >> 4);
-          if (32 * (sl + u) >= nr) break;
-          if (nr - 32 * (sl + u) < 32) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              d[u][e] = e < valid ? d[u][e] : uint16_t(0);
-#pragma unroll
-              for (int j = 0; j < JT; ++j) xs[u][j][e] = e < valid ? xs[u][j][e] : uint16_t(0);
-            }
-          }
-#pragma unroll
-          for (int j = 0; j < JT; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, d[u]),
-                                                             __builtin_bit_cast(bf16x8_t, xs[u][j]), acc[j], 0, 0, 0);
-        }
+        for (int j = 0; j < JT; ++j) o.x[j][e] = e < valid ? o.x[j][e] : uint16_t(0);
       }
     }
 #pragma unroll
     for (int j = 0; j < JT; ++j)
+      c[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, o.d),
+                                                     __builtin_bit_cast(bf16x8_t, o.x[j]), c[j], 0, 0, 0);
+  };
+  constexpr int kRound = SR > 2 ? SR : 2;
+  Operands o[kRound];
+  if (rs.slices == 1 && SR > 1) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) part[wave + 8 * k][4 * (lane >> 4) + r][16 * j + (lane & 15)] = acc[j][r];
+    for (int k = 0; k < SR; ++k) o[k] = request(wave + 8 * k, 0);
+#pragma unroll
+    for (int k = 0; k < SR; ++k) products(wave + 8 * k, 0, o[k], acc[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < SR; ++k)
+      for (int sl = 0; sl < rs.slices; sl += kRound) {
+#pragma unroll
+        for (int u = 0; u < kRound; ++u) o[u] = request(wave + 8 * k, sl + u);
+#pragma unroll
+        for (int u = 0; u < kRound; ++u)
+          if (sl + u < rs.slices) products(wave + 8 * k, sl + u, o[u], acc[k]);
+      }
   }
+#pragma unroll
+  for (int k = 0; k < SR; ++k)
+#pragma unroll
+    for (int j = 0; j < JT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) part[wave + 8 * k][4 * (lane >> 4) + r][16 * j + (lane & 15)] = acc[k][j][r];
   lds_barrier();
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {

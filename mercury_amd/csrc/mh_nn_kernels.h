@@ -1,8 +1,10 @@
-// mh_nn_kernels.h -- device kernels shared by the surrogate networks
-// (mlp.hip, cnn.hip): a matrix-core GEMM (bf16 operands, FP32 accumulate)
-// with bias/GELU epilogues, the squared-error loss gradient, fixed-order column sums (bias
-// gradients), split-K weight gradients, Adam, and small helpers.  Every reduction runs in a fixed
-// order, so training is deterministic.
+// mh_nn_kernels.h -- arithmetic and helpers shared by the surrogate networks
+// (mlp.hip, cnn.hip, mh_dense.h), and the layer-by-layer kernels of
+// perceptrons wider or deeper than mh_dense.h takes: a matrix-core GEMM (bf16
+// operands, FP32 accumulate) with bias/GELU epilogues, the squared-error loss
+// gradient, fixed-order column sums (bias gradients), split-K weight
+// gradients and Adam.  Every reduction runs in a fixed order, so training is
+// deterministic.
 //
 // gelu(x) = 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))).  Adam follows
 // Kingma & Ba (2015), Algorithm 1 (bias-corrected moments).
@@ -118,9 +120,8 @@ __device__ __forceinline__ u16x8_t bits8(const Raw8<__hip_bfloat16>& r) { return
 // Operand loaders of the matrix-core tile: A(m, k) and B(k, n) return the
 // bf16 bits of op(A)[m][k] and op(B)[k][n] (callers stay within M, N and
 // the k range).  kContigK says which index is contiguous in memory (k, or
-// m / n), so a tile's elements are read along it.  A loader with kVec8
-// also reads 8 consecutive elements along that index in one call,
-// vec8(a, b), with (a, b) the first element's indices in the order of
+// m / n), so a tile's elements are read along it, 8 consecutive ones in one
+// call, vec8(a, b), with (a, b) the first element's indices in the order of
 // operator(); callers use it only when all 8 lie inside the operand.
 //   StridedA: op(A)[m][k] = TR ? p[k*ld + m] : p[m*ld + k]
 //   StridedB: op(B)[k][n] = TR ? p[n*ld + k] : p[k*ld + n]
@@ -129,7 +130,6 @@ struct StridedA {
   const T* p;
   int ld;
   static constexpr bool kContigK = !TR;
-  static constexpr bool kVec8 = true;
   __device__ uint16_t operator()(int m, int k) const {
     return TR ? ld_bf16(p, static_cast<size_t>(k) * ld + m) : ld_bf16(p, static_cast<size_t>(m) * ld + k);
   }
@@ -147,7 +147,6 @@ struct StridedB {
   const T* p;
   int ld;
   static constexpr bool kContigK = TR;
-  static constexpr bool kVec8 = true;
   __device__ uint16_t operator()(int k, int n) const {
     return TR ? ld_bf16(p, static_cast<size_t>(n) * ld + k) : ld_bf16(p, static_cast<size_t>(k) * ld + n);
   }
@@ -190,50 +189,31 @@ __device__ __forceinline__ auto raw_at(const L& l, int r0, int k0) {
 template <bool IS_A, typename L>
 __device__ __forceinline__ u16x8_t fetch_slice(const L& l, int ROWS, int r0, int k0, int k_end) {
   u16x8_t v;
-  if constexpr (L::kVec8) {
-    if constexpr (L::kContigK) {
-      const int r = r0 + (threadIdx.x >> 2), k = k0 + ((threadIdx.x & 3) << 3);
-      if (r < ROWS && k + 8 <= k_end) v = vec8_at<IS_A>(l, r, k);
-      else {
+  if constexpr (L::kContigK) {
+    const int r = r0 + (threadIdx.x >> 2), k = k0 + ((threadIdx.x & 3) << 3);
+    if (r < ROWS && k + 8 <= k_end) v = vec8_at<IS_A>(l, r, k);
+    else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (r < ROWS && k + j < k_end) ? load_at<IS_A>(l, r, k + j) : uint16_t(0);
-      }
-    } else {
-      const int r = r0 + ((threadIdx.x & 7) << 3), k = k0 + (threadIdx.x >> 3);
-      if (r + 8 <= ROWS && k < k_end) v = vec8_at<IS_A>(l, r, k);
-      else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (r + j < ROWS && k < k_end) ? load_at<IS_A>(l, r + j, k) : uint16_t(0);
-      }
+      for (int j = 0; j < 8; ++j) v[j] = (r < ROWS && k + j < k_end) ? load_at<IS_A>(l, r, k + j) : uint16_t(0);
     }
   } else {
+    const int r = r0 + ((threadIdx.x & 7) << 3), k = k0 + (threadIdx.x >> 3);
+    if (r + 8 <= ROWS && k < k_end) v = vec8_at<IS_A>(l, r, k);
+    else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int e = threadIdx.x + 256 * j;
-      const int rr = L::kContigK ? e / 32 : e % 64, kk = L::kContigK ? e % 32 : e / 64;
-      const int r = r0 + rr, k = k0 + kk;
-      v[j] = (r < ROWS && k < k_end) ? load_at<IS_A>(l, r, k) : uint16_t(0);
+      for (int j = 0; j < 8; ++j) v[j] = (r + j < ROWS && k < k_end) ? load_at<IS_A>(l, r + j, k) : uint16_t(0);
     }
   }
   return v;
 }
 template <typename L>
 __device__ __forceinline__ void put_slice(u16x8_t v, uint16_t (*s)[40]) {
-  if constexpr (L::kVec8) {
-    if constexpr (L::kContigK) {
-      *reinterpret_cast<u16x8_t*>(&s[threadIdx.x >> 2][(threadIdx.x & 3) << 3]) = v;
-    } else {
-      const int kk = threadIdx.x >> 3, rr = (threadIdx.x & 7) << 3;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) s[rr + j][kk] = v[j];
-    }
+  if constexpr (L::kContigK) {
+    *reinterpret_cast<u16x8_t*>(&s[threadIdx.x >> 2][(threadIdx.x & 3) << 3]) = v;
   } else {
+    const int kk = threadIdx.x >> 3, rr = (threadIdx.x & 7) << 3;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int e = threadIdx.x + 256 * j;
-      if constexpr (L::kContigK) s[e / 32][e % 32] = v[j];
-      else s[e % 64][e / 64] = v[j];
-    }
+    for (int j = 0; j < 8; ++j) s[rr + j][kk] = v[j];
   }
 }
 
@@ -254,10 +234,8 @@ __device__ __forceinline__ void put_slice(u16x8_t v, uint16_t (*s)[40]) {
 // order on every path and every run.
 constexpr int kMk = 32;                  // k per slice
 constexpr int kMRow = kMk + 8;           // LDS row pitch in bf16 (80 B, 16 B aligned)
-// slices per step: 2 for the dense layers' GEMMs (k of 64 or 256); the
-// convolution kernels' gathered operands take one (a deeper stage lowers
-// their occupancy without shortening them)
-constexpr int kStageDense = 2, kStageConv = 1, kStageWgrad = 1;
+// slices per step: 2 for the GEMMs of activations, 1 for weight gradients
+constexpr int kStageDense = 2, kStageWgrad = 1;
 template <int S, bool FAST, typename LA, typename LB>
 __device__ __forceinline__ void mfma_tile(const LA& la, const LB& lb, int M, int N, int k_begin, int k_end, int m0,
                                           int n0, uint16_t (*sa)[kTile][kMRow], uint16_t (*sb)[kTile][kMRow],
@@ -375,21 +353,8 @@ __device__ __forceinline__ void mfma_store(const f32x4_t (&acc)[2][2], float* __
       }
 }
 
-// C[M x N] = op(A) op(B) (bf16 products, fp32 sums) with loaders la, lb,
-// then epilogue EPI.
-template <typename LA, typename LB, int EPI>
-__global__ __launch_bounds__(256) void gemm_l(LA la, LB lb, float* __restrict__ C, int ldc, int M, int N, int K,
-                                              const float* __restrict__ bias, float* __restrict__ Z,
-                                              const float* __restrict__ Zprev) {
-  __shared__ __align__(16) uint16_t sa[kStageConv][kTile][kMRow];
-  __shared__ __align__(16) uint16_t sb[kStageConv][kTile][kMRow];
-  const int m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile;
-  f32x4_t acc[2][2];
-  mfma_tile<kStageConv, false>(la, lb, M, N, 0, K, m0, n0, sa, sb, acc);
-  mfma_store<EPI>(acc, C, ldc, M, N, m0, n0, bias, Z, Zprev);
-}
-
-// The same for strided operands: op(A)[m][k] = TRA ? A[k*lda + m] :
+// C[M x N] = op(A) op(B) (bf16 products, fp32 sums) of strided operands, then
+// epilogue EPI: op(A)[m][k] = TRA ? A[k*lda + m] :
 // A[m*lda + k], op(B)[k][n] = TRB ? B[n*ldb + k] : B[k*ldb + n].
 template <typename TA, typename TB, bool TRA, bool TRB, int EPI>
 __global__ __launch_bounds__(256) void gemm(const TA* __restrict__ A, int lda, const TB* __restrict__ B,
