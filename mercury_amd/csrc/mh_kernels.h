@@ -94,6 +94,17 @@ __host__ __device__ inline int pos_slots(int n) { return n + (n >> 3) + 1; }
 #endif
 __host__ __device__ constexpr int mass_slot(int i) { return i + (i >> MH_MASS_SKEW_SHIFT); }
 __host__ __device__ constexpr int mass_slots(int block) { return block + (block >> MH_MASS_SKEW_SHIFT) + 1; }
+// The mass-parallel kernels' lane of the mass with the rank-th most records
+// of n: groups of 64 ranks (a wave's worth, so its lists have similar
+// lengths) go to waves 0, 1, 2, 3, 7, 6, 5, 4, 8, .. -- waves of a workgroup
+// are dealt to the CU's four SIMDs in turn, so the plain order gave SIMD 0
+// the longest list of every four waves: 64 of 227 wave-records of an 8^3
+// robot (58 this way).  A group of four waves that is not full keeps its
+// order (lanes are dense).
+__host__ __device__ constexpr int mass_lane(int rank, int n) {
+  const int four = rank >> 8;
+  return (four & 1) && (four + 1) * 256 <= n ? (rank & ~255) | ((~rank) & 192) | (rank & 63) : rank;
+}
 // Mass-parallel kernels: distinct (rest length, material) pairs per pack;
 // the LDS pair tables hold kMassPairMax, the last one reserved for padding
 // records.  Per pair: {L, k} (float2; L the actuated rest length), {1/k,

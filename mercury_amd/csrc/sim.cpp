@@ -672,6 +672,10 @@ void upload_mass(mh_sim* s, Part& part, std::vector<uint16_t>& perm, std::vector
       if (gather && fill_p[x] != fill_p[y]) return fill_p[x] > fill_p[y];
       return tx > ty;
     });
+    {
+      const std::vector<uint32_t> ranked(order);
+      for (uint32_t i = 0; i < nm; i++) order[mass_lane(static_cast<int>(i), static_cast<int>(nm))] = ranked[i];
+    }
     for (uint32_t i = 0; i < nm; i++) {
       perm[d.mass_begin + i] = static_cast<uint16_t>(order[i]);
       lane[order[i]] = i;

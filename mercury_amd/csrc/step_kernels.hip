@@ -863,8 +863,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE))) vo
 // length}.  Each substep the
 // lanes below the pair count compute the next substep's L of one pair each
 // (the actuation once per pair instead of once per spring).  Lanes take
-// masses in the order of p.mperm (most records first, so a wave's lists
-// have similar lengths).  Each lane keeps its records in registers: one
+// masses in the order of p.mperm (groups of 64 by record count, so a wave's
+// lists have similar lengths; mass_lane).  Each lane keeps its records in registers: one
 // record per spring of its mass, in ascending spring index (a spring from
 // the mass to itself twice), padded to the wave's longest list with
 // records of the null pair (last entry: stiffness 0 for force, +inf for
@@ -911,10 +911,11 @@ __device__ __forceinline__ void mass_pairs_init(unsigned char* smem, const StepP
 }
 
 // The next substep's actuated rest lengths: L(t) of every pair into the
-// first word of its dyn entry (STRIDE words per entry).
+// first word of its dyn entry (STRIDE words per entry).  From the last lane
+// down: the last waves have the shortest record lists, or none.
 template <int BLOCK, int STRIDE = 2>
 __device__ __forceinline__ void mass_pairs_advance(unsigned char* smem, int n_pairs, int dyn, int cst, float t) {
-  for (int i = static_cast<int>(threadIdx.x); i < n_pairs; i += BLOCK) {
+  for (int i = BLOCK - 1 - static_cast<int>(threadIdx.x); i < n_pairs; i += BLOCK) {
     const float4 cs = reinterpret_cast<const float4*>(smem + cst)[i];
     reinterpret_cast<float*>(smem + dyn)[STRIDE * i] = fmaf(cs.w, actuation(cs.x, cs.y, cs.z, t), cs.w);
   }

@@ -192,6 +192,7 @@ __global__ __launch_bounds__(kVoxThreads) void voxel_population(VoxelBuildParams
       const uint16_t kj = key[j];
       rank += (kj > mine) | ((kj == mine) & (j < tid));
     }
+    rank = mass_lane(rank, n);
     lane_of[tid] = static_cast<uint16_t>(rank);
     p.mperm[static_cast<size_t>(r) * n + rank] = static_cast<uint16_t>(tid);
   }
