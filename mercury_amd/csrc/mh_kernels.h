@@ -75,6 +75,7 @@ struct KernelVariant {
   int mpt;        // masses per thread
   const void* fn; // kernel symbol
   const void* fn_stress = nullptr;  // variant used when stress is tracked (null: fn)
+  const void* fn_wide = nullptr;    // variant for at most one workgroup per CU (null: fn); same results
 };
 
 // All compiled variants (table lives in step_kernels.hip).
@@ -157,7 +158,7 @@ constexpr int kMStreamMats = 256;
 constexpr int kMStream6Mats = 16;
 size_t lds_bytes_mstream(int block, int mpt);
 
-hipError_t launch_step(const KernelVariant& v, int n_packs, size_t lds_bytes,
+hipError_t launch_step(const KernelVariant& v, int n_packs, size_t lds_bytes, int compute_units,
                        hipStream_t stream, const StepParams& p);
 
 // Start time of each of the ceil(n_steps / K) launches of a call into

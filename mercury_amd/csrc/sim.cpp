@@ -120,6 +120,7 @@ struct mh_sim {
   hipStream_t aux = nullptr;         // second part of a mixed plan
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   int lds_limit = mh::kMaxLdsBytes;
+  int compute_units = 0;
 
   // population (host copies used for packing and collect)
   int n_robots = 0;
@@ -831,7 +832,7 @@ void upload_plan(mh_sim* s, Plan& plan) {
     // dynamic LDS above 64 KB needs the attribute (the mass-parallel
     // streaming kernel's LDS is static)
     if (part.lds > 64 * 1024 && !(part.v->kind == MH_KERNEL_STREAM && part.v->chunked == 2)) {
-      for (const void* fn : {part.v->fn, part.v->fn_stress})
+      for (const void* fn : {part.v->fn, part.v->fn_stress, part.v->fn_wide})
         if (fn)
           (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(part.lds));
     }
@@ -962,7 +963,8 @@ int issue(mh_sim* s, int n_steps, int track) {
     for (int done = 0; done < n_steps;) {
       const int n = std::min(K, n_steps - done);
       StepParams p = make_params(s, part, launches, n, track);
-      hip_check(launch_step(*part.v, static_cast<int>(part.packs.size()), part.lds, st, p), "step launch");
+      hip_check(launch_step(*part.v, static_cast<int>(part.packs.size()), part.lds, s->compute_units, st, p),
+                "step launch");
       done += n;
       launches++;
     }
@@ -1114,6 +1116,8 @@ int mh_sim_create(const mh_config* cfg, const mh_material_set* set, mh_sim** out
   if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, cfg->device) == hipSuccess &&
       lds > 0)
     s->lds_limit = std::min(lds, mh::kMaxLdsBytes);
+  mh::hip_check(hipDeviceGetAttribute(&s->compute_units, hipDeviceAttributeMultiprocessorCount, cfg->device),
+                "device attribute");
   mh::hip_check(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), "stream");
   mh::hip_check(hipStreamCreateWithFlags(&s->aux, hipStreamNonBlocking), "stream");
   mh::hip_check(hipEventCreateWithFlags(&s->ev_fork, hipEventDisableTiming), "event");
@@ -1558,7 +1562,7 @@ int mh_sim_set_voxel_population(mh_sim* s, int n_robots, int nx, int ny, int nz,
     part.lds = mh::lds_bytes_mass(v->block, s->composite_count);
     part.n_robots = R;
     if (part.lds > 64 * 1024)
-      for (const void* fn : {v->fn, v->fn_stress})
+      for (const void* fn : {v->fn, v->fn_stress, v->fn_wide})
         if (fn) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(part.lds));
     plan.parts.push_back(std::move(part));
   }

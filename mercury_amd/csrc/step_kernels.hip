@@ -995,9 +995,84 @@ __device__ __forceinline__ void mass_substep(unsigned char* smem, const StepPara
   __syncthreads();
 }
 
+// The force solver's substep for launches that leave at most one workgroup
+// to a CU: with three waves or fewer per SIMD a wave's own chain is what
+// takes the time (per record an LDS read, 130 cycles, and 20 dependent
+// operations), so U records are evaluated together, with one fast-path test
+// and the next U already read from LDS, and the decoded addresses stay in
+// registers.  Records past the wave's longest list are padding, whose terms
+// are signed zeros.  Same operations and order per record, same bits.
+constexpr int wide_slots(int maxp, int u) { return (2 * maxp + u - 1) / u * u; }
+template <int BLOCK, int MAXP, int U, int CUR>
+__device__ __forceinline__ void mass_substep_wide(unsigned char* smem, const StepParams& p, MassState& ms,
+                                                  const uint32_t (&po)[wide_slots(MAXP, U)],
+                                                  const uint32_t (&pa)[wide_slots(MAXP, U)], int nr_w, bool live, int pslot, int n_pairs, float t) {
+  constexpr int kP0 = kMassPos + CUR * mass_pos_bytes<BLOCK>();
+  constexpr int kP1 = kMassPos + (1 - CUR) * mass_pos_bytes<BLOCK>();
+  constexpr int kPairs = mass_pair_base(BLOCK, 2);
+  constexpr int kD0 = kPairs + CUR * kMassDynBytes;
+  constexpr int kD1 = kPairs + (1 - CUR) * kMassDynBytes;
+  constexpr int kCst = kPairs + 3 * kMassDynBytes;
+  constexpr int kBatches = wide_slots(MAXP, U) / U;
+  float4 other[2][U];
+  float2 Lk[2][U];
+  auto read = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      other[b & 1][i] = *reinterpret_cast<const float4*>(smem + kP0 + po[U * b + i]);
+      Lk[b & 1][i] = *reinterpret_cast<const float2*>(smem + kD0 + pa[U * b + i]);
+    }
+  };
+  const float4 own = live ? *reinterpret_cast<const float4*>(smem + kP0 + 16 * pslot)
+                          : make_float4(0.f, 0.f, 0.f, 0.f);
+  read(0);
+  float ax = 0.0f, ay = 0.0f, az = 0.0f;
+#pragma unroll
+  for (int b = 0; b < kBatches; ++b) {
+    if (U * b < nr_w) {
+      if (b + 1 < kBatches) read(b + 1);
+      float dx[U], dy[U], dz[U], s[U], f[U];
+      bool fast = true;
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const float4 o = other[b & 1][i];
+        dx[i] = own.x - o.x;
+        dy[i] = own.y - o.y;
+        dz[i] = own.z - o.z;
+        s[i] = sum_sq3(dx[i], dy[i], dz[i]);
+        fast = fast && s[i] >= kLenFastLo;
+        keep_b128(o.w);
+      }
+      if (__builtin_amdgcn_ballot_w64(fast) == __builtin_amdgcn_read_exec()) {
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+          const float d = sqrt_rn_inrange(s[i]);
+          f[i] = (Lk[b & 1][i].y * (Lk[b & 1][i].x - d)) * rcp_rn_inrange(d);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+          const float d = sqrtf(s[i]);
+          f[i] = (Lk[b & 1][i].y * (Lk[b & 1][i].x - d)) * (1.0f / (d + kEps));
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        ax = fmaf(f[i], dx[i], ax);
+        ay = fmaf(f[i], dy[i], ay);
+        az = fmaf(f[i], dz[i], az);
+      }
+    }
+  }
+  if (live) *reinterpret_cast<float4*>(smem + kP1 + 16 * pslot) = integrate<MH_SOLVER_FORCE>(ms, ax, ay, az, p);
+  mass_pairs_advance<BLOCK>(smem, n_pairs, kD1, kCst, t + p.dt);
+  __syncthreads();
+}
+
 // STRESS (xpbd only) accumulates per-spring stress; the variant without it
-// frees 2 MAXP registers per lane.
-template <int SOLVER, int BLOCK, int MAXP, bool STRESS>
+// frees 2 MAXP registers per lane.  WIDE > 0 (force only): mass_substep_wide
+// with batches of WIDE records.
+template <int SOLVER, int BLOCK, int MAXP, bool STRESS, int WIDE = 0>
 __global__ __launch_bounds__(BLOCK) void step_mass(StepParams p) {
   extern __shared__ __align__(16) unsigned char smem[];
   const PackDesc d = p.packs[blockIdx.x];
@@ -1057,13 +1132,35 @@ __global__ __launch_bounds__(BLOCK) void step_mass(StepParams p) {
 
   // substeps in pairs, so each buffer's base is a constant offset
   int step = 0;
-  for (; step + 1 < p.n_steps; step += 2) {
+  if constexpr (WIDE > 0) {
+    static_assert(SOLVER == MH_SOLVER_FORCE, "the wide substep serves the force solver");
+    constexpr int kSlots = wide_slots(MAXP, WIDE > 0 ? WIDE : 1);
+    uint32_t po[kSlots], pa[kSlots];
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+      const uint32_t r = k < 2 * MAXP ? rr[k < 2 * MAXP ? k : 0] : pad;
+      po[k] = r & 0xffffu;
+      pa[k] = r >> 16;
+    }
+    nr_w = __builtin_amdgcn_readfirstlane(nr_w);
+    for (; step + 1 < p.n_steps; step += 2) {
+      mass_substep_wide<BLOCK, MAXP, WIDE, 0>(smem, p, ms, po, pa, nr_w, live, pslot, n_pairs, t);
+      t = t + p.dt;
+      mass_substep_wide<BLOCK, MAXP, WIDE, 1>(smem, p, ms, po, pa, nr_w, live, pslot, n_pairs, t);
+      t = t + p.dt;
+    }
+    if (step < p.n_steps) {
+      mass_substep_wide<BLOCK, MAXP, WIDE, 0>(smem, p, ms, po, pa, nr_w, live, pslot, n_pairs, t);
+      ++step;
+    }
+  }
+  for (; WIDE == 0 && step + 1 < p.n_steps; step += 2) {
     mass_substep<SOLVER, BLOCK, MAXP, STRESS, 0>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, n_pairs, t);
     t = t + p.dt;
     mass_substep<SOLVER, BLOCK, MAXP, STRESS, 1>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, n_pairs, t);
     t = t + p.dt;
   }
-  if (step < p.n_steps)
+  if (WIDE == 0 && step < p.n_steps)
     mass_substep<SOLVER, BLOCK, MAXP, STRESS, 0>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, n_pairs, t);
 
   if (live) {
@@ -1310,11 +1407,25 @@ __global__ void robot_com(const float4* pos, const uint8_t* mass_id, const uint3
   out[3 * r + 2] = cz;
 }
 
+// step_mass for at most one workgroup per CU (force solver).  MI355X, us per
+// substep of the evaluate call, plain -> wide: one robot of 125 masses
+// (256-lane block, batches of 4) 3.4 -> 2.4, 256 of 343 masses (512) 4.8 ->
+// 3.8, one of 729 (768, batches of 2) 3.5 -> 3.2, 256 of them 5.5 -> 5.1.
+// 100 robots of 1000 masses (1024, batches of 2) went from 5.0 to 5.5: four
+// waves per SIMD cover the latency, so that block has none.
+template <int SOLVER, int B, int P>
+const void* wide_mass() {
+  if constexpr (SOLVER == MH_SOLVER_FORCE && B < 1024)
+    return reinterpret_cast<const void*>(&step_mass<SOLVER, B, P, false, B <= 512 ? 4 : 2>);
+  return nullptr;
+}
+
 #define MH_LDS(SOLVER, B, S, M) \
   {SOLVER, MH_KERNEL_LDS, 0, B, S, M, reinterpret_cast<const void*>(&step_lds<SOLVER, B, S, M>)}
 #define MH_MASS(SOLVER, B, P)                                                         \
   {SOLVER, MH_KERNEL_MASS, 0, B, P, 1, reinterpret_cast<const void*>(&step_mass<SOLVER, B, P, false>), \
-   reinterpret_cast<const void*>(&step_mass<SOLVER, B, P, (SOLVER == MH_SOLVER_XPBD_REF)>)}
+   reinterpret_cast<const void*>(&step_mass<SOLVER, B, P, (SOLVER == MH_SOLVER_XPBD_REF)>), \
+   wide_mass<SOLVER, B, P>()}
 #define MH_MASSG(SOLVER, B, P)                                                        \
   {SOLVER, MH_KERNEL_MASS, 1, B, P, 1, reinterpret_cast<const void*>(&step_massg<SOLVER, B, P, false>), \
    reinterpret_cast<const void*>(&step_massg<SOLVER, B, P, (SOLVER == MH_SOLVER_XPBD_REF)>)}
@@ -1392,11 +1503,12 @@ size_t lds_bytes_stream(int mass_cap, int n_mat) {
   return 16u * static_cast<size_t>(mass_cap) + 4u * static_cast<size_t>(n_mat);
 }
 
-hipError_t launch_step(const KernelVariant& v, int n_packs, size_t lds_bytes, hipStream_t stream,
+hipError_t launch_step(const KernelVariant& v, int n_packs, size_t lds_bytes, int compute_units, hipStream_t stream,
                        const StepParams& p) {
   StepParams args = p;
   void* kargs[] = {&args};
   const void* fn = (p.track_stress && v.fn_stress) ? v.fn_stress : v.fn;
+  if (v.fn_wide && n_packs <= compute_units) fn = v.fn_wide;
   // the mass-parallel streaming kernel's LDS is a static array
   const size_t dyn = (v.kind == MH_KERNEL_STREAM && v.chunked == 2) ? 0 : lds_bytes;
   return hipLaunchKernel(fn, dim3(n_packs), dim3(v.block), kargs, dyn, stream);
