@@ -207,6 +207,9 @@ struct VoxelBuildParams {
 };
 hipError_t launch_voxel_population(const VoxelBuildParams& p, int n_robots, hipStream_t stream);
 
+// The first three words of each float4, packed (positions, velocities).
+hipError_t launch_xyz(const float4* src, float* dst, size_t n, hipStream_t stream);
+
 // Per-robot COM of non-air masses (SoftBody::updateCOM order).
 hipError_t launch_com(const float4* pos, const uint8_t* mass_id,
                       const uint32_t* robot_mass_begin, int n_robots,

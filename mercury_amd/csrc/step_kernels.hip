@@ -1387,6 +1387,13 @@ __global__ void set_clock(float* times, float t0, float dt, int n_steps, int K) 
   }
 }
 
+// {x, y, z, w} -> {x, y, z}, one lane per word written, for copies straight
+// into a caller's array; the copy to the host that follows bounds it.
+__global__ void pack_xyz(const float* __restrict__ src, float* __restrict__ dst, size_t words) {
+  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < words) dst[i] = src[4 * (i / 3) + i % 3];
+}
+
 // ------------------------------------------------------------------ COM
 __global__ void robot_com(const float4* pos, const uint8_t* mass_id, const uint32_t* begin,
                           int n_robots, float* out) {
@@ -1516,6 +1523,14 @@ hipError_t launch_step(const KernelVariant& v, int n_packs, size_t lds_bytes, in
 
 hipError_t launch_clock(float* times, float t0, float dt, int n_steps, int K, hipStream_t stream) {
   hipLaunchKernelGGL(set_clock, dim3(1), dim3(64), 0, stream, times, t0, dt, n_steps, K);
+  return hipGetLastError();
+}
+
+hipError_t launch_xyz(const float4* src, float* dst, size_t n, hipStream_t stream) {
+  const size_t blocks = (3 * n + 255) / 256;
+  if (blocks > 0x7fffffffu) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(pack_xyz, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream,
+                     reinterpret_cast<const float*>(src), dst, 3 * n);
   return hipGetLastError();
 }
 
