@@ -75,7 +75,11 @@ struct KernelVariant {
   int mpt;        // masses per thread
   const void* fn; // kernel symbol
   const void* fn_stress = nullptr;  // variant used when stress is tracked (null: fn)
-  const void* fn_wide = nullptr;    // variant for at most one workgroup per CU (null: fn); same results
+  // variants for launches that leave the SIMDs short of waves, with the same
+  // results (null: none): at most one workgroup per CU (step_mass), packs of
+  // few masses (step_massg, which has one for tracked stresses too)
+  const void* fn_wide = nullptr;
+  const void* fn_wide_stress = nullptr;
 };
 
 // All compiled variants (table lives in step_kernels.hip).

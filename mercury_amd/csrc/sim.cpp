@@ -834,7 +834,7 @@ void upload_plan(mh_sim* s, Plan& plan) {
     // dynamic LDS above 64 KB needs the attribute (the mass-parallel
     // streaming kernel's LDS is static)
     if (part.lds > 64 * 1024 && !(part.v->kind == MH_KERNEL_STREAM && part.v->chunked == 2)) {
-      for (const void* fn : {part.v->fn, part.v->fn_stress, part.v->fn_wide})
+      for (const void* fn : {part.v->fn, part.v->fn_stress, part.v->fn_wide, part.v->fn_wide_stress})
         if (fn)
           (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(part.lds));
     }
@@ -1569,7 +1569,7 @@ int mh_sim_set_voxel_population(mh_sim* s, int n_robots, int nx, int ny, int nz,
     part.lds = mh::lds_bytes_mass(v->block, s->composite_count);
     part.n_robots = R;
     if (part.lds > 64 * 1024)
-      for (const void* fn : {v->fn, v->fn_stress, v->fn_wide})
+      for (const void* fn : {v->fn, v->fn_stress, v->fn_wide, v->fn_wide_stress})
         if (fn) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(part.lds));
     plan.parts.push_back(std::move(part));
   }

@@ -1176,6 +1176,15 @@ __global__ __launch_bounds__(BLOCK) void step_mass(StepParams p) {
   }
 }
 
+// Packs of at most this many masses take step_massg's wide form: with one
+// workgroup per CU that is two live waves per SIMD or fewer, and a wave's own
+// chain of LDS reads takes the time.  With three the LDS pipe is busy and the
+// batches cost 1-4 %.  MI355X, ms per 1000 untracked substeps, plain and
+// wide: one robot of 125 masses 3.79 and 2.84, of 343 3.88 and 3.20, of 512
+// 4.03 and 3.76, of 729 4.48 and 4.65; 512 robots of 512 masses 8.21 and
+// 7.84, of 686 masses per pack 4.48 and 4.62, of 729 9.15 and 9.50.
+constexpr int kWideMaxMasses = 512;
+
 // XPBD term of the gather kernel.  fast_ok says that the workgroup's
 // positions and the pack's materials lie where div_rn_from_rcp is exact
 // (coordinates 0 or of magnitude in [2^-56, 2^20]; stiffness divisor in
@@ -1213,6 +1222,43 @@ __device__ __forceinline__ void xpbd_term_L(float4 pa, float4 pb, float L, float
   cz = lambda * nz;
 }
 
+// The terms of the first n <= N of a batch of records, e = {L, k, 1/k, rest
+// length}, with one fast-path test for all of them.  Same results as
+// xpbd_term_L: its two paths agree wherever the short one is taken.
+template <int N>
+__device__ __forceinline__ void xpbd_terms(float4 pa, const float4 (&pb)[N], const float4 (&e)[N], int n,
+                                           bool fast_ok, float (&cx)[N], float (&cy)[N], float (&cz)[N],
+                                           float (&lambda)[N]) {
+  float dx[N], dy[N], dz[N], s[N];
+  bool fast = fast_ok;
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+    if (u < n) {
+      dx[u] = pa.x - pb[u].x;
+      dy[u] = pa.y - pb[u].y;
+      dz[u] = pa.z - pb[u].z;
+      s[u] = sum_sq3(dx[u], dy[u], dz[u]);
+      fast = fast && __float_as_uint(s[u]) - __float_as_uint(kLenFastLo) <=
+                         __float_as_uint(kSqrtFastHi) - __float_as_uint(kLenFastLo);
+    }
+  if (__builtin_amdgcn_ballot_w64(fast) == __builtin_amdgcn_read_exec()) {
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (u < n) {
+        const float d = sqrt_rn_inrange(s[u]);
+        const float y = rcp_rn_inrange(d);
+        lambda[u] = div_rn_from_rcp(-(d - e[u].x), e[u].y, e[u].z);
+        cx[u] = lambda[u] * div_rn_from_rcp(dx[u], d, y);
+        cy[u] = lambda[u] * div_rn_from_rcp(dy[u], d, y);
+        cz[u] = lambda[u] * div_rn_from_rcp(dz[u], d, y);
+      }
+  } else {
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+      if (u < n) xpbd_term_L(pa, pb[u], e[u].x, e[u].y, e[u].z, false, cx[u], cy[u], cz[u], lambda[u]);
+  }
+}
+
 // Position of a mass in the fast division's range: each coordinate 0 or of
 // magnitude in [2^-56, 2^20] (NaN is not).
 __device__ __forceinline__ bool position_in_div_range(float4 q) {
@@ -1245,7 +1291,9 @@ __device__ __forceinline__ bool position_in_div_range(float4 q) {
 // entries).  XPBD: the
 // flags (one per substep parity) record whether any position written for
 // that substep left the fast division's range.
-template <int SOLVER, int BLOCK, int MAXP, bool STRESS>
+// WIDE: two records and four entries at a time, the next ones' LDS reads
+// ahead of the arithmetic, for packs of at most kWideMaxMasses masses.
+template <int SOLVER, int BLOCK, int MAXP, bool STRESS, bool WIDE>
 __global__ __launch_bounds__(BLOCK) void step_massg(StepParams p) {
   static_assert(SOLVER == MH_SOLVER_XPBD_REF,
                 "step_massg stores 12-byte terms: the xpbd step only (the force step_mass is faster)");
@@ -1321,34 +1369,109 @@ __global__ __launch_bounds__(BLOCK) void step_massg(StepParams p) {
       fast_ok = p.fast_div && s_flag[step & 1] == 0u;
       if (tid == 0) s_flag[(step + 1) & 1] = 0u;  // read last in the previous substep
     }
+    if constexpr (WIDE) {
+      constexpr int kB = 2;
+      float4 no[kB], nl[kB];
+      auto fetch = [&](int k0) {
 #pragma unroll
-    for (int k = 0; k < MAXP; ++k) {
-      if (k < np_w) {
-        const uint32_t r = rp[k];
-        const float4 other = *reinterpret_cast<const float4*>(smem + kMassPos + (r & 0xffffu));
-        float cx, cy, cz, lambda;
-        const float4 e = *reinterpret_cast<const float4*>(smem + kDyn + (r >> 16));  // {L, k, 1/k, rest}
-        xpbd_term_L(own, other, e.x, e.y, e.z, fast_ok, cx, cy, cz, lambda);
-        keep_b128(other.w);
-        keep_b128(e.w);
-        if (STRESS && k < np) st[k] = st[k] + lambda / e.w;
-        float* slot = reinterpret_cast<float*>(mine + 12 * k);
-        slot[0] = cx;
-        slot[1] = cy;
-        slot[2] = cz;
+        for (int u = 0; u < kB; ++u)
+          if (k0 + u < MAXP) {  // records from np_w on are the null pair's
+            const uint32_t r = rp[k0 + u];
+            no[u] = *reinterpret_cast<const float4*>(smem + kMassPos + (r & 0xffffu));
+            nl[u] = *reinterpret_cast<const float4*>(smem + kDyn + (r >> 16));  // {L, k, 1/k, rest}
+          }
+      };
+      fetch(0);
+#pragma unroll
+      for (int k0 = 0; k0 < MAXP; k0 += kB) {
+        if (k0 < np_w) {
+          float4 other[kB], e[kB];
+          float cx[kB], cy[kB], cz[kB], lambda[kB];
+#pragma unroll
+          for (int u = 0; u < kB; ++u) {
+            other[u] = no[u];
+            e[u] = nl[u];
+          }
+          fetch(k0 + kB);
+          xpbd_terms<kB>(own, other, e, min(kB, MAXP - k0), fast_ok, cx, cy, cz, lambda);
+#pragma unroll
+          for (int u = 0; u < kB; ++u)
+            if (k0 + u < MAXP) {
+              keep_b128(other[u].w);
+              keep_b128(e[u].w);
+              if (STRESS && k0 + u < np) st[k0 + u] = st[k0 + u] + lambda[u] / e[u].w;
+              float* slot = reinterpret_cast<float*>(mine + 12 * (k0 + u));
+              slot[0] = cx[u];
+              slot[1] = cy[u];
+              slot[2] = cz[u];
+            }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < MAXP; ++k) {
+        if (k < np_w) {
+          const uint32_t r = rp[k];
+          const float4 other = *reinterpret_cast<const float4*>(smem + kMassPos + (r & 0xffffu));
+          float cx, cy, cz, lambda;
+          const float4 e = *reinterpret_cast<const float4*>(smem + kDyn + (r >> 16));  // {L, k, 1/k, rest}
+          xpbd_term_L(own, other, e.x, e.y, e.z, fast_ok, cx, cy, cz, lambda);
+          keep_b128(other.w);
+          keep_b128(e.w);
+          if (STRESS && k < np) st[k] = st[k] + lambda / e.w;
+          float* slot = reinterpret_cast<float*>(mine + 12 * k);
+          slot[0] = cx;
+          slot[1] = cy;
+          slot[2] = cz;
+        }
       }
     }
     __syncthreads();
     float ax = 0.0f, ay = 0.0f, az = 0.0f;
+    if constexpr (WIDE) {
+      constexpr int kB = 4;
+      float nq[kB][3];
+      auto gather = [&](int k0) {
 #pragma unroll
-    for (int k = 0; k < 2 * MAXP; ++k) {
-      if (k < ne_w) {
-        const uint32_t e = re[k];
-        const float* q = reinterpret_cast<const float*>(smem + (e & ~1u));
-        const float sg = __uint_as_float(0x3f800000u | (e << 31));
-        ax = fmaf(q[0], sg, ax);
-        ay = fmaf(q[1], sg, ay);
-        az = fmaf(q[2], sg, az);
+        for (int u = 0; u < kB; ++u)
+          if (k0 + u < 2 * MAXP) {
+            const float* q = reinterpret_cast<const float*>(smem + (re[k0 + u] & ~1u));
+            nq[u][0] = q[0];
+            nq[u][1] = q[1];
+            nq[u][2] = q[2];
+          }
+      };
+      gather(0);
+#pragma unroll
+      for (int k0 = 0; k0 < 2 * MAXP; k0 += kB) {
+        if (k0 < ne_w) {
+          float q[kB][3];
+#pragma unroll
+          for (int u = 0; u < kB; ++u)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) q[u][c] = nq[u][c];
+          gather(k0 + kB);
+#pragma unroll
+          for (int u = 0; u < kB; ++u)
+            if (k0 + u < 2 * MAXP) {  // entries from ne_w on are the zero term
+              const float sg = __uint_as_float(0x3f800000u | (re[k0 + u] << 31));
+              ax = fmaf(q[u][0], sg, ax);
+              ay = fmaf(q[u][1], sg, ay);
+              az = fmaf(q[u][2], sg, az);
+            }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 2 * MAXP; ++k) {
+        if (k < ne_w) {
+          const uint32_t e = re[k];
+          const float* q = reinterpret_cast<const float*>(smem + (e & ~1u));
+          const float sg = __uint_as_float(0x3f800000u | (e << 31));
+          ax = fmaf(q[0], sg, ax);
+          ay = fmaf(q[1], sg, ay);
+          az = fmaf(q[2], sg, az);
+        }
       }
     }
     if (live) {
@@ -1429,13 +1552,24 @@ const void* wide_mass() {
 
 #define MH_LDS(SOLVER, B, S, M) \
   {SOLVER, MH_KERNEL_LDS, 0, B, S, M, reinterpret_cast<const void*>(&step_lds<SOLVER, B, S, M>)}
+// step_massg's wide form, for the 768-lane block the plans use (one workgroup
+// per CU; in the smaller blocks its registers would cost resident waves).
+template <int SOLVER, int BLOCK, int MAXP, bool STRESS>
+const void* wide_massg() {
+  if constexpr (BLOCK == 768)
+    return reinterpret_cast<const void*>(&step_massg<SOLVER, BLOCK, MAXP, STRESS, true>);
+  else
+    return nullptr;
+}
+
 #define MH_MASS(SOLVER, B, P)                                                         \
   {SOLVER, MH_KERNEL_MASS, 0, B, P, 1, reinterpret_cast<const void*>(&step_mass<SOLVER, B, P, false>), \
    reinterpret_cast<const void*>(&step_mass<SOLVER, B, P, (SOLVER == MH_SOLVER_XPBD_REF)>), \
    wide_mass<SOLVER, B, P>()}
 #define MH_MASSG(SOLVER, B, P)                                                        \
-  {SOLVER, MH_KERNEL_MASS, 1, B, P, 1, reinterpret_cast<const void*>(&step_massg<SOLVER, B, P, false>), \
-   reinterpret_cast<const void*>(&step_massg<SOLVER, B, P, (SOLVER == MH_SOLVER_XPBD_REF)>)}
+  {SOLVER, MH_KERNEL_MASS, 1, B, P, 1, reinterpret_cast<const void*>(&step_massg<SOLVER, B, P, false, false>), \
+   reinterpret_cast<const void*>(&step_massg<SOLVER, B, P, (SOLVER == MH_SOLVER_XPBD_REF), false>), \
+   wide_massg<SOLVER, B, P, false>(), wide_massg<SOLVER, B, P, true>()}
 #define MH_CHUNK(SOLVER, B, M) \
   {SOLVER, MH_KERNEL_STREAM, 1, B, 0, M, reinterpret_cast<const void*>(&step_chunk<SOLVER, B, M>)}
 #define MH_STREAM(SOLVER, B) \
@@ -1515,7 +1649,11 @@ hipError_t launch_step(const KernelVariant& v, int n_packs, size_t lds_bytes, in
   StepParams args = p;
   void* kargs[] = {&args};
   const void* fn = (p.track_stress && v.fn_stress) ? v.fn_stress : v.fn;
-  if (v.fn_wide && n_packs <= compute_units) fn = v.fn_wide;
+  if (v.kind == MH_KERNEL_MASS && v.chunked == 1) {
+    if (v.fn_wide && p.mass_cap <= kWideMaxMasses) fn = p.track_stress ? v.fn_wide_stress : v.fn_wide;
+  } else if (v.fn_wide && n_packs <= compute_units) {
+    fn = v.fn_wide;
+  }
   // the mass-parallel streaming kernel's LDS is a static array
   const size_t dyn = (v.kind == MH_KERNEL_STREAM && v.chunked == 2) ? 0 : lds_bytes;
   return hipLaunchKernel(fn, dim3(n_packs), dim3(v.block), kargs, dyn, stream);
