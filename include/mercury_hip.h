@@ -320,12 +320,13 @@ int mh_mlp_forward(mh_mlp* net, const float* x, int batch, float* y);
  * (code under HIP graph capture, serving loops that score offspring every
  * generation): mh_mlp_forward on device buffers x [batch x in] and
  * y [batch x out], enqueued on `stream` (a hipStream_t; NULL = the
- * network's own stream) without waiting, with the same results.  Networks
- * of up to 4 layers of at most 256 units keep their hidden activations on
- * chip; wider ones use a fixed device array of MH_MLP_SCRATCH_FLOATS floats
- * (16 MiB on each device the library runs on, held until the process
- * ends), used in two halves.  For every network batch x (widest hidden
- * layer) over MH_MLP_SCRATCH_FLOATS / 2 gives MH_ERR_RANGE and launches nothing.  All
+ * network's own stream) without waiting, with the same results.  y may
+ * overlap x where the network has a hidden layer.  Hidden activations use a
+ * fixed device array of MH_MLP_SCRATCH_FLOATS floats (16 MiB on each device
+ * the library runs on, held until the process ends) in two halves, or stay
+ * on chip (networks of up to 4 layers of at most 256 units, where y does not
+ * overlap x).  For every network batch x (widest hidden layer) over
+ * MH_MLP_SCRATCH_FLOATS / 2 gives MH_ERR_RANGE and launches nothing.  All
  * calls on one device share the array, so calls that overlap in time there
  * (other streams, other threads) race; training the same network
  * concurrently races too.  Calls no hipMalloc, hipFree or allocating

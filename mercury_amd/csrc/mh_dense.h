@@ -63,10 +63,12 @@ __device__ __forceinline__ void pack_store(const PackedLayer& p, uint16_t* pack,
   pack[p.bwd + packed_index(k * p.out + o, c, (p.c + 15) >> 4)] = b;
 }
 
-__global__ void pack_layer(PackedLayer p, const float* params, uint16_t* pack) {
+// plain (may be null): the bf16 weights as they lie in the parameter vector
+__global__ void pack_layer(PackedLayer p, const float* params, uint16_t* pack, uint16_t* plain) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= p.out * p.in) return;
   pack_store(p, pack, e / p.in, e % p.in, params[p.w_off + e]);
+  if (plain) plain[p.w_off + e] = bf16_bits(params[p.w_off + e]);
 }
 
 __global__ void fill_zero_u16(uint16_t* p, int n) {
@@ -391,7 +393,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_net(DenseShape sh, const 
 
 struct AdamArgs {
   float *p, *m, *v;
-  uint16_t* pack;
+  uint16_t *pack, *plain;  // as pack_layer's
   float lr, b1, b2, eps, bc1, bc2;
 };
 
@@ -589,7 +591,10 @@ __global__ __launch_bounds__(kWgThreads) void dense_wgrad(DenseShape sh, DenseTr
     for (int s = 0; s < kSplits; ++s)
       if (s < rs.splits) g += part[s][r][c];
     const float w = finish(p.w_off + o * p.in + i, g, pmv[k]);
-    if constexpr (ADAM) pack_store(p, ad.pack, o, i, w);
+    if constexpr (ADAM) {
+      pack_store(p, ad.pack, o, i, w);
+      if (ad.plain) ad.plain[p.w_off + o * p.in + i] = bf16_bits(w);
+    }
   }
 }
 

@@ -52,7 +52,7 @@ struct mh_mlp {
   Dev<uint16_t> pack;         // fused: bf16 weights in the kernels' operand order
   std::vector<Dev<uint16_t>> X16, D16;  // fused: weight-gradient operands of a batch
   std::vector<Dev<float>> delta;        // fused: gradients of every layer's output
-  Dev<__hip_bfloat16> w16;    // otherwise: bf16 copy of the whole parameter vector (weights used)
+  Dev<__hip_bfloat16> w16;    // bf16 copy of the parameter vector for the layer-by-layer kernels (weights used)
   std::vector<Dev<float>> Z, A, dA;  // per layer activations / gradients
   Dev<float> x, t, dY, terms, data_x, data_t;
   Dev<float> epoch_terms;     // loss terms of every batch of a training run's last epoch
@@ -120,13 +120,24 @@ void refresh_weights(mh_mlp* net) {
     for (int l = 0; l < net->L(); l++) {
       const PackedLayer& p = net->shape.layer[l];
       hipLaunchKernelGGL(pack_layer, dim3((p.out * p.in + 255) / 256), dim3(256), 0, net->stream, p, net->params.p,
-                         net->pack.p);
+                         net->pack.p, reinterpret_cast<uint16_t*>(net->w16.p));
     }
   } else {
     hipLaunchKernelGGL(to_bf16, dim3((net->n_params + 255) / 256), dim3(256), 0, net->stream, net->params.p,
                        net->w16.p, static_cast<int>(net->n_params));
   }
   hipcheck(hipGetLastError(), "weights");
+}
+
+// Whether a forward pass on device buffers that may not allocate takes the
+// layer-by-layer kernels though the network is fused: y overlaps x, and a
+// fused workgroup would write rows that another still reads (the layers' last
+// kernel starts when all of x has been read).
+bool forward_by_layers(const mh_mlp* net, const float* x, int B, const float* y) {
+  const size_t nx = static_cast<size_t>(B) * net->sizes.front() * sizeof(float),
+               ny = static_cast<size_t>(B) * net->sizes.back() * sizeof(float);
+  const uintptr_t ax = reinterpret_cast<uintptr_t>(x), ay = reinterpret_cast<uintptr_t>(y);
+  return net->L() > 1 && ax < ay + ny && ay < ax + nx;
 }
 
 // Fused forward of B rows on the device, x -> y.  A workgroup reads every
@@ -309,8 +320,8 @@ int mh_mlp_create(int device, int n_layers, const int* sizes, uint64_t seed, mh_
       for (int l = 0; l < n_layers; l++) widest = std::max<size_t>(widest, static_cast<size_t>(sizes[l]) * sizes[l + 1]);
       // split partials of one tensor, or of every parameter for adam_step_splits
       net->part.ensure(static_cast<size_t>(kMlpSplit) * std::max(widest, net->n_params));
-      net->w16.ensure(off);
     }
+    net->w16.ensure(off);
     // He-uniform weights (bound sqrt(6 / fan_in)), zero biases
     std::mt19937_64 rng(seed);
     std::vector<float> p(off, 0.f);
@@ -433,7 +444,7 @@ int mh_mlp_forward_noalloc(mh_mlp* net, const float* x, int batch, float* y, voi
                                         std::to_string(half) + " floats)");
     hipcheck(hipSetDevice(net->device), "hipSetDevice");
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : net->stream;
-    if (net->fused) {
+    if (net->fused && !forward_by_layers(net, x, batch, y)) {
       fused_forward(net, x, batch, y, s);
       return MH_OK;
     }
@@ -517,7 +528,8 @@ int mh_mlp_train(mh_mlp* net, const float* x, const float* target, int n, int ba
         const float bc2 = 1.f - std::pow(b2, static_cast<float>(net->adam_t));
         if (last) batches++;
         if (net->fused) {
-          const AdamArgs adam{net->params.p, net->m.p, net->v.p, net->pack.p, lr, b1, b2, eps, bc1, bc2};
+          const AdamArgs adam{net->params.p, net->m.p, net->v.p, net->pack.p,
+                              reinterpret_cast<uint16_t*>(net->w16.p), lr, b1, b2, eps, bc1, bc2};
           fused_backward(net, net->data_x.p, net->data_t.p, net->idx.p + b0, batch, terms, &adam);
           continue;
         }
