@@ -55,9 +55,13 @@ __device__ __forceinline__ int packed_index(int k, int n, int n_tiles) {
   return (((k >> 5) * n_tiles + (n >> 4)) * 64 + ((k & 31) >> 3) * 16 + (n & 15)) * 8 + (k & 7);
 }
 
+// A weight as bf16: round to nearest even, NaN stays NaN (bf16_bits takes
+// finite values only).
+__device__ __forceinline__ uint16_t weight_bits(float w) { return __builtin_bit_cast(uint16_t, __float2bfloat16(w)); }
+
 // Stores weight (o, i) in both packings.
 __device__ __forceinline__ void pack_store(const PackedLayer& p, uint16_t* pack, int o, int i, float w) {
-  const uint16_t b = bf16_bits(w);
+  const uint16_t b = weight_bits(w);
   pack[p.fwd + packed_index(i, o, (p.out + 15) >> 4)] = b;
   const int k = i / p.c, c = i - k * p.c;
   pack[p.bwd + packed_index(k * p.out + o, c, (p.c + 15) >> 4)] = b;
@@ -68,7 +72,7 @@ __global__ void pack_layer(PackedLayer p, const float* params, uint16_t* pack, u
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= p.out * p.in) return;
   pack_store(p, pack, e / p.in, e % p.in, params[p.w_off + e]);
-  if (plain) plain[p.w_off + e] = bf16_bits(params[p.w_off + e]);
+  if (plain) plain[p.w_off + e] = weight_bits(params[p.w_off + e]);
 }
 
 __global__ void fill_zero_u16(uint16_t* p, int n) {
@@ -593,7 +597,7 @@ __global__ __launch_bounds__(kWgThreads) void dense_wgrad(DenseShape sh, DenseTr
     const float w = finish(p.w_off + o * p.in + i, g, pmv[k]);
     if constexpr (ADAM) {
       pack_store(p, ad.pack, o, i, w);
-      if (ad.plain) ad.plain[p.w_off + o * p.in + i] = bf16_bits(w);
+      if (ad.plain) ad.plain[p.w_off + o * p.in + i] = weight_bits(w);
     }
   }
 }
