@@ -1000,8 +1000,8 @@ __device__ __forceinline__ void mass_substep(unsigned char* smem, const StepPara
 // takes the time (per record an LDS read, 130 cycles, and 20 dependent
 // operations), so U records are evaluated together, with one fast-path test
 // and the next U already read from LDS, and the decoded addresses stay in
-// registers.  Records past the wave's longest list are padding, whose terms
-// are signed zeros.  Same operations and order per record, same bits.
+// registers.  Records past the wave's longest list add signed zeros.  Same
+// operations and order per record, same bits.
 constexpr int wide_slots(int maxp, int u) { return (2 * maxp + u - 1) / u * u; }
 template <int BLOCK, int MAXP, int U, int CUR>
 __device__ __forceinline__ void mass_substep_wide(unsigned char* smem, const StepParams& p, MassState& ms,
@@ -1135,14 +1135,18 @@ __global__ __launch_bounds__(BLOCK) void step_mass(StepParams p) {
   if constexpr (WIDE > 0) {
     static_assert(SOLVER == MH_SOLVER_FORCE, "the wide substep serves the force solver");
     constexpr int kSlots = wide_slots(MAXP, WIDE > 0 ? WIDE : 1);
-    uint32_t po[kSlots], pa[kSlots];
+    nr_w = __builtin_amdgcn_readfirstlane(nr_w);
+    // Records from nr_w on fill the last batch.  They are of the null pair at
+    // the position of the lane's last record, not at the ghost, whose squared
+    // distance overflows from 1.8e19 on, and 0 times infinity is no signed
+    // zero: a filler's term is one wherever the last record's is finite.
+    uint32_t po[kSlots], pa[kSlots], last = pad;
 #pragma unroll
     for (int k = 0; k < kSlots; ++k) {
-      const uint32_t r = k < 2 * MAXP ? rr[k < 2 * MAXP ? k : 0] : pad;
-      po[k] = r & 0xffffu;
-      pa[k] = r >> 16;
+      if (k < 2 * MAXP && k < nr_w) last = rr[k < 2 * MAXP ? k : 0];
+      po[k] = last & 0xffffu;
+      pa[k] = (k < nr_w ? last : pad) >> 16;
     }
-    nr_w = __builtin_amdgcn_readfirstlane(nr_w);
     for (; step + 1 < p.n_steps; step += 2) {
       mass_substep_wide<BLOCK, MAXP, WIDE, 0>(smem, p, ms, po, pa, nr_w, live, pslot, n_pairs, t);
       t = t + p.dt;
