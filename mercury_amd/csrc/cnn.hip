@@ -1185,7 +1185,7 @@ int mh_cnn_train(mh_cnn* net, const uint8_t* genomes, const float* target, int n
         net->adam_t++;
         const float bc1 = 1.f - std::pow(b1, static_cast<float>(net->adam_t));
         const float bc2 = 1.f - std::pow(b2, static_cast<float>(net->adam_t));
-        const AdamArgs adam{net->params.p, net->m.p, net->v.p, net->pack.p, nullptr, lr, b1, b2, eps, bc1, bc2};
+        const AdamArgs adam{net->params.p, net->m.p, net->v.p, net->pack.p, lr, b1, b2, eps, bc1, bc2};
         loss_backward_to(net, net->data_g.p, net->data_t.p, net->idx.p + b0, batch,
                          last ? net->epoch_terms.p + static_cast<size_t>(batches) * batch : net->terms.p, &adam);
         if (last) batches++;

@@ -55,9 +55,11 @@ __device__ __forceinline__ int packed_index(int k, int n, int n_tiles) {
   return (((k >> 5) * n_tiles + (n >> 4)) * 64 + ((k & 31) >> 3) * 16 + (n & 15)) * 8 + (k & 7);
 }
 
-// A weight as bf16: round to nearest even, NaN stays NaN (bf16_bits takes
+// A weight as bf16: round to nearest even, and NaN stays NaN (bf16_bits takes
 // finite values only).
-__device__ __forceinline__ uint16_t weight_bits(float w) { return __builtin_bit_cast(uint16_t, __float2bfloat16(w)); }
+__device__ __forceinline__ uint16_t weight_bits(float w) {
+  return w != w ? static_cast<uint16_t>(__float_as_uint(w) >> 16 | 0x40u) : bf16_bits(w);
+}
 
 // Stores weight (o, i) in both packings.
 __device__ __forceinline__ void pack_store(const PackedLayer& p, uint16_t* pack, int o, int i, float w) {
@@ -261,7 +263,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_net(DenseShape sh, const 
     }
     *reinterpret_cast<u16x8_t*>(&act[0][r][k]) = v;
   }
-  if (L > 1) fetch(1, 0, kSlices);
+  if (kStages > 1) fetch(1, 0, kSlices);
   // operands for the stores at the end: every layer's input and output
   // gradient
   uint2 xo[TRAIN ? L : 1][T], go[TRAIN ? L : 1][T];
@@ -397,7 +399,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_net(DenseShape sh, const 
 
 struct AdamArgs {
   float *p, *m, *v;
-  uint16_t *pack, *plain;  // as pack_layer's
+  uint16_t* pack;
   float lr, b1, b2, eps, bc1, bc2;
 };
 
@@ -595,10 +597,7 @@ __global__ __launch_bounds__(kWgThreads) void dense_wgrad(DenseShape sh, DenseTr
     for (int s = 0; s < kSplits; ++s)
       if (s < rs.splits) g += part[s][r][c];
     const float w = finish(p.w_off + o * p.in + i, g, pmv[k]);
-    if constexpr (ADAM) {
-      pack_store(p, ad.pack, o, i, w);
-      if (ad.plain) ad.plain[p.w_off + o * p.in + i] = weight_bits(w);
-    }
+    if constexpr (ADAM) pack_store(p, ad.pack, o, i, w);
   }
 }
 

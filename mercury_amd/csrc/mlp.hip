@@ -528,8 +528,7 @@ int mh_mlp_train(mh_mlp* net, const float* x, const float* target, int n, int ba
         const float bc2 = 1.f - std::pow(b2, static_cast<float>(net->adam_t));
         if (last) batches++;
         if (net->fused) {
-          const AdamArgs adam{net->params.p, net->m.p, net->v.p, net->pack.p,
-                              reinterpret_cast<uint16_t*>(net->w16.p), lr, b1, b2, eps, bc1, bc2};
+          const AdamArgs adam{net->params.p, net->m.p, net->v.p, net->pack.p, lr, b1, b2, eps, bc1, bc2};
           fused_backward(net, net->data_x.p, net->data_t.p, net->idx.p + b0, batch, terms, &adam);
           continue;
         }
@@ -547,6 +546,10 @@ int mh_mlp_train(mh_mlp* net, const float* x, const float* target, int n, int ba
         hipcheck(hipGetLastError(), "train step");
       }
     }
+    // the fused update keeps the packed weights only
+    if (net->fused && n_epochs > 0)
+      hipLaunchKernelGGL(to_bf16, dim3((net->n_params + 255) / 256), dim3(256), 0, net->stream, net->params.p,
+                         net->w16.p, static_cast<int>(net->n_params));
     // the last epoch's mean over batches of each batch's summed terms / batch
     std::vector<float> terms(static_cast<size_t>(batches) * nt);
     if (batches)
