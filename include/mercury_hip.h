@@ -324,8 +324,8 @@ int mh_mlp_forward(mh_mlp* net, const float* x, int batch, float* y);
  * overlap x where the network has a hidden layer.  Hidden activations use a
  * fixed device array of MH_MLP_SCRATCH_FLOATS floats (16 MiB on each device
  * the library runs on, held until the process ends) in two halves, or stay
- * on chip (networks of up to 4 layers of at most 256 units, where y does not
- * overlap x).  For every network batch x (widest hidden layer) over
+ * on chip (networks of up to 4 layers of at most 256 units, where that is
+ * faster and y does not overlap x).  For every network batch x (widest hidden layer) over
  * MH_MLP_SCRATCH_FLOATS / 2 gives MH_ERR_RANGE and launches nothing.  All
  * calls on one device share the array, so calls that overlap in time there
  * (other streams, other threads) race; training the same network

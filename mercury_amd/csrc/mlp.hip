@@ -11,7 +11,8 @@
 //
 // Networks of up to kDenseMaxLayers layers of at most kDenseMaxWidth units
 // (the surrogate is 64-256-256-1) run as the fused kernels of mh_dense.h:
-// one launch forward, two per training step.  Wider ones run a launch per
+// one launch forward, two per training step.  Wider ones, and large batches of
+// narrow ones on device buffers (forward_by_layers), run a launch per
 // layer and direction: 64x64 output tiles, 256 threads (four waves of 2x2
 // 16x16 MFMA blocks), K in steps of 32 staged through LDS as bf16.  Weight
 // gradients reduce over the batch in row splits whose partials are summed in
@@ -130,14 +131,29 @@ void refresh_weights(mh_mlp* net) {
 }
 
 // Whether a forward pass on device buffers that may not allocate takes the
-// layer-by-layer kernels though the network is fused: y overlaps x, and a
-// fused workgroup would write rows that another still reads (the layers' last
-// kernel starts when all of x has been read).
+// layer-by-layer kernels though the network is fused.
 bool forward_by_layers(const mh_mlp* net, const float* x, int B, const float* y) {
-  const size_t nx = static_cast<size_t>(B) * net->sizes.front() * sizeof(float),
-               ny = static_cast<size_t>(B) * net->sizes.back() * sizeof(float);
+  const int L = net->L(), in = net->sizes.front(), out = net->sizes.back();
+  // y overlaps x: a fused workgroup would write rows that another still reads
+  // (the layers' last kernel starts when all of x has been read)
+  const size_t nx = static_cast<size_t>(B) * in * sizeof(float), ny = static_cast<size_t>(B) * out * sizeof(float);
   const uintptr_t ax = reinterpret_cast<uintptr_t>(x), ay = reinterpret_cast<uintptr_t>(y);
-  return net->L() > 1 && ax < ay + ny && ay < ax + nx;
+  if (L > 1 && ax < ay + ny && ay < ax + nx) return true;
+  // Large batches of narrow networks: the fused kernel computes 256 units a
+  // layer whatever the width (0.16 ns per row and layer once the chip is full),
+  // the layers' kernels have one launch per layer (about 5 us) and then the
+  // time of their own widths.  MI355X, us fused and by layers: 8-8-1 at 16384
+  // rows 10.7 and 10.8, at 65536 37 and 12; 64-64-64-1 at 16384 15.7 and 18.6,
+  // at 32768 29.5 and 21; 32-100-1 at 20480 20.0 and 18.3.  One layer: 64-1 at
+  // 8192 rows 4.3 and 4.4, at 12288 5.7 and 4.4, at 65536 12.3 and 5.6; 64-256
+  // at 16384 9.9 and 8.0, at 24576 12.5 and 12.8; 128-128 at 24576 9.6 and
+  // 8.4, at 32768 10.5 and 11.1; 128-256 at 12288 9.0 and 8.5, at 16384 10.0
+  // and 11.0; 256-1 at 65536 16.0 and 16.9.  (Networks of a hidden layer of 128
+  // units or more stay under 16384 rows: the scratch array's limit.)
+  if (L > 1) return B > 16384;
+  // (one layer of 128 x 128 and more: fused from 4.1e8 products on)
+  const size_t macs = static_cast<size_t>(in) * out;
+  return B > 8192 && in < 256 && (macs < 128 * 128 || macs * B <= 410000000u);
 }
 
 // Fused forward of B rows on the device, x -> y.  A workgroup reads every
