@@ -80,6 +80,17 @@ struct KernelVariant {
   // few masses (step_massg, which has one for tracked stresses too)
   const void* fn_wide = nullptr;
   const void* fn_wide_stress = nullptr;
+  // step_massg variants for packs whose last waves have few records
+  const void* fn_uneven = nullptr;
+  const void* fn_uneven_stress = nullptr;
+};
+
+// What launch_step chooses a variant's kernel by, with the same results.
+struct LaunchShape {
+  int n_packs;
+  size_t lds_bytes;
+  int compute_units;
+  bool uneven;  // mass-parallel: in most packs the last wave with masses has at most half the first's records
 };
 
 // All compiled variants (table lives in step_kernels.hip).
@@ -162,8 +173,7 @@ constexpr int kMStreamMats = 256;
 constexpr int kMStream6Mats = 16;
 size_t lds_bytes_mstream(int block, int mpt);
 
-hipError_t launch_step(const KernelVariant& v, int n_packs, size_t lds_bytes, int compute_units,
-                       hipStream_t stream, const StepParams& p);
+hipError_t launch_step(const KernelVariant& v, const LaunchShape& l, hipStream_t stream, const StepParams& p);
 
 // Start time of each of the ceil(n_steps / K) launches of a call into
 // times[], by the reference's float recurrence t += dt from t0 (one lane;

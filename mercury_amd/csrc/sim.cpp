@@ -98,6 +98,7 @@ struct Part {
   size_t lds = 0;
   uint32_t pack_offset = 0;         // first descriptor in the device array
   int n_robots = 0;
+  bool uneven = false;              // LaunchShape::uneven
 };
 
 // Robots that fit the LDS kernel go to the LDS part, the rest to the
@@ -641,6 +642,7 @@ void upload_mass(mh_sim* s, Part& part, std::vector<uint16_t>& perm, std::vector
   mrec.resize(rec_end, 0u);
   mcnt.resize(cnt_end);
   // pass 2 (packs in parallel): pairs, lane order and records
+  std::atomic<size_t> n_uneven{0};
   parallel_for(n_packs, [&](size_t pi) {
     const PackDesc& d = part.packs[pi];
     const std::vector<uint64_t>& table = tables[pi];
@@ -737,7 +739,14 @@ void upload_mass(mh_sim* s, Part& part, std::vector<uint16_t>& perm, std::vector
       cnt[2 * i] = static_cast<uint8_t>(gather ? fill_p[order[i]] : fill[order[i]]);
       cnt[2 * i + 1] = static_cast<uint8_t>(gather ? fill[order[i]] : 0u);
     }
+    auto longest = [cnt](uint32_t lane0, uint32_t lane1) {
+      uint8_t n = 0;
+      for (uint32_t i = lane0; i < lane1; i++) n = std::max(n, cnt[2 * i]);
+      return n;
+    };
+    if (nm && 2 * longest((nm - 1) & ~63u, nm) <= longest(0, std::min(nm, 64u))) n_uneven++;
   });
+  part.uneven = 2 * n_uneven > n_packs;
   std::stable_sort(part.packs.begin(), part.packs.end(), [](const PackDesc& x, const PackDesc& y) {
     return static_cast<uint64_t>(x.n_spring) + x.n_mass > static_cast<uint64_t>(y.n_spring) + y.n_mass;
   });
@@ -834,7 +843,8 @@ void upload_plan(mh_sim* s, Plan& plan) {
     // dynamic LDS above 64 KB needs the attribute (the mass-parallel
     // streaming kernel's LDS is static)
     if (part.lds > 64 * 1024 && !(part.v->kind == MH_KERNEL_STREAM && part.v->chunked == 2)) {
-      for (const void* fn : {part.v->fn, part.v->fn_stress, part.v->fn_wide, part.v->fn_wide_stress})
+      for (const void* fn : {part.v->fn, part.v->fn_stress, part.v->fn_wide, part.v->fn_wide_stress,
+                             part.v->fn_uneven, part.v->fn_uneven_stress})
         if (fn)
           (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(part.lds));
     }
@@ -965,8 +975,8 @@ int issue(mh_sim* s, int n_steps, int track) {
     for (int done = 0; done < n_steps;) {
       const int n = std::min(K, n_steps - done);
       StepParams p = make_params(s, part, launches, n, track);
-      hip_check(launch_step(*part.v, static_cast<int>(part.packs.size()), part.lds, s->compute_units, st, p),
-                "step launch");
+      const LaunchShape shape{static_cast<int>(part.packs.size()), part.lds, s->compute_units, part.uneven};
+      hip_check(launch_step(*part.v, shape, st, p), "step launch");
       done += n;
       launches++;
     }
@@ -1569,7 +1579,7 @@ int mh_sim_set_voxel_population(mh_sim* s, int n_robots, int nx, int ny, int nz,
     part.lds = mh::lds_bytes_mass(v->block, s->composite_count);
     part.n_robots = R;
     if (part.lds > 64 * 1024)
-      for (const void* fn : {v->fn, v->fn_stress, v->fn_wide, v->fn_wide_stress})
+      for (const void* fn : {v->fn, v->fn_stress, v->fn_wide, v->fn_wide_stress, v->fn_uneven, v->fn_uneven_stress})
         if (fn) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(part.lds));
     plan.parts.push_back(std::move(part));
   }

@@ -911,14 +911,39 @@ __device__ __forceinline__ void mass_pairs_init(unsigned char* smem, const StepP
 }
 
 // The next substep's actuated rest lengths: L(t) of every pair into the
-// first word of its dyn entry (STRIDE words per entry).  From the last lane
-// down: the last waves have the shortest record lists, or none.
+// first word of its dyn entry (STRIDE words per entry).  first: this lane's
+// first pair (pair_order).
 template <int BLOCK, int STRIDE = 2>
-__device__ __forceinline__ void mass_pairs_advance(unsigned char* smem, int n_pairs, int dyn, int cst, float t) {
-  for (int i = BLOCK - 1 - static_cast<int>(threadIdx.x); i < n_pairs; i += BLOCK) {
+__device__ __forceinline__ void mass_pairs_advance(unsigned char* smem, int first, int n_pairs, int dyn, int cst,
+                                                   float t) {
+  for (int i = first; i < n_pairs; i += BLOCK) {
     const float4 cs = reinterpret_cast<const float4*>(smem + cst)[i];
     reinterpret_cast<float*>(smem + dyn)[STRIDE * i] = fmaf(cs.w, actuation(cs.x, cs.y, cs.z, t), cs.w);
   }
+}
+
+// The lane's first pair in mass_pairs_advance: pairs go to the lanes from the
+// last one down where the last waves have less to do than the first (lists at
+// most half as long, or no masses), else from the first lane up -- the oldest
+// waves are issued first, so equally loaded last waves end the substep, and
+// the pairs' sine after them adds to it.  MI355X, us per substep on the last
+// lanes and on the first: one voxel robot of 125 masses 2.21 and 2.32, 600 of
+// 512 masses 6.86 and 7.10; lists of equal length and no idle wave (760 masses
+// in 768 lanes), 2 springs each 0.98 and 0.91, 6 springs 1.49 and 1.38, 600
+// such robots 3.30 and 3.17.  `longest` is the wave's longest list; the
+// workgroup reads the result after the next barrier.
+constexpr int kMassLists = kMassZero + 32;  // longest list of the first wave and of the last with masses
+__device__ __forceinline__ void pair_order_put(unsigned char* smem, int nm, int longest) {
+  const int tid = static_cast<int>(threadIdx.x);
+  int* lists = reinterpret_cast<int*>(smem + kMassLists);
+  if (tid == 0) lists[0] = longest;
+  if (tid == ((max(nm, 1) - 1) & ~63)) lists[1] = longest;
+}
+template <int BLOCK>
+__device__ __forceinline__ int pair_order_get(const unsigned char* smem, int nm) {
+  const int* lists = reinterpret_cast<const int*>(smem + kMassLists);
+  const int tid = static_cast<int>(threadIdx.x);
+  return 2 * lists[1] <= lists[0] || nm <= BLOCK - 64 ? BLOCK - 1 - tid : tid;
 }
 
 // step_massg's pair table: one float4 {L(t), k, 1/k, rest length} per pair
@@ -947,8 +972,8 @@ __device__ __forceinline__ void massg_pairs_init(unsigned char* smem, const Step
 template <int SOLVER, int BLOCK, int MAXP, bool STRESS, int CUR>
 __device__ __forceinline__ void mass_substep(unsigned char* smem, const StepParams& p, MassState& ms,
                                              uint32_t (&rr)[2 * MAXP], float (&st)[STRESS ? 2 * MAXP : 1],
-                                             uint32_t first, int nr, int nr_w, bool live, int pslot, int n_pairs,
-                                             float t) {
+                                             uint32_t first, int nr, int nr_w, bool live, int pslot, int pair0,
+                                             int n_pairs, float t) {
   constexpr int kP0 = kMassPos + CUR * mass_pos_bytes<BLOCK>();
   constexpr int kP1 = kMassPos + (1 - CUR) * mass_pos_bytes<BLOCK>();
   constexpr int kPairs = mass_pair_base(BLOCK, 2);
@@ -991,7 +1016,7 @@ __device__ __forceinline__ void mass_substep(unsigned char* smem, const StepPara
     __builtin_amdgcn_sched_barrier(0);
   }
   if (live) *reinterpret_cast<float4*>(smem + kP1 + 16 * pslot) = integrate<SOLVER>(ms, ax, ay, az, p);
-  mass_pairs_advance<BLOCK>(smem, n_pairs, kD1, kCst, t + p.dt);
+  mass_pairs_advance<BLOCK>(smem, pair0, n_pairs, kD1, kCst, t + p.dt);
   __syncthreads();
 }
 
@@ -1006,7 +1031,8 @@ constexpr int wide_slots(int maxp, int u) { return (2 * maxp + u - 1) / u * u; }
 template <int BLOCK, int MAXP, int U, int CUR>
 __device__ __forceinline__ void mass_substep_wide(unsigned char* smem, const StepParams& p, MassState& ms,
                                                   const uint32_t (&po)[wide_slots(MAXP, U)],
-                                                  const uint32_t (&pa)[wide_slots(MAXP, U)], int nr_w, bool live, int pslot, int n_pairs, float t) {
+                                                  const uint32_t (&pa)[wide_slots(MAXP, U)], int nr_w, bool live, int pslot,
+                                                  int pair0, int n_pairs, float t) {
   constexpr int kP0 = kMassPos + CUR * mass_pos_bytes<BLOCK>();
   constexpr int kP1 = kMassPos + (1 - CUR) * mass_pos_bytes<BLOCK>();
   constexpr int kPairs = mass_pair_base(BLOCK, 2);
@@ -1065,7 +1091,7 @@ __device__ __forceinline__ void mass_substep_wide(unsigned char* smem, const Ste
     }
   }
   if (live) *reinterpret_cast<float4*>(smem + kP1 + 16 * pslot) = integrate<MH_SOLVER_FORCE>(ms, ax, ay, az, p);
-  mass_pairs_advance<BLOCK>(smem, n_pairs, kD1, kCst, t + p.dt);
+  mass_pairs_advance<BLOCK>(smem, pair0, n_pairs, kD1, kCst, t + p.dt);
   __syncthreads();
 }
 
@@ -1128,7 +1154,9 @@ __global__ __launch_bounds__(BLOCK) void step_mass(StepParams p) {
   // wave-wide loop bound
   int nr_w = nr;
   for (int off = 32; off > 0; off >>= 1) nr_w = max(nr_w, __shfl_xor(nr_w, off));
+  pair_order_put(smem, nm, nr_w);
   __syncthreads();
+  const int pair0 = pair_order_get<BLOCK>(smem, nm);
 
   // substeps in pairs, so each buffer's base is a constant offset
   int step = 0;
@@ -1148,24 +1176,24 @@ __global__ __launch_bounds__(BLOCK) void step_mass(StepParams p) {
       pa[k] = (k < nr_w ? last : pad) >> 16;
     }
     for (; step + 1 < p.n_steps; step += 2) {
-      mass_substep_wide<BLOCK, MAXP, WIDE, 0>(smem, p, ms, po, pa, nr_w, live, pslot, n_pairs, t);
+      mass_substep_wide<BLOCK, MAXP, WIDE, 0>(smem, p, ms, po, pa, nr_w, live, pslot, pair0, n_pairs, t);
       t = t + p.dt;
-      mass_substep_wide<BLOCK, MAXP, WIDE, 1>(smem, p, ms, po, pa, nr_w, live, pslot, n_pairs, t);
+      mass_substep_wide<BLOCK, MAXP, WIDE, 1>(smem, p, ms, po, pa, nr_w, live, pslot, pair0, n_pairs, t);
       t = t + p.dt;
     }
     if (step < p.n_steps) {
-      mass_substep_wide<BLOCK, MAXP, WIDE, 0>(smem, p, ms, po, pa, nr_w, live, pslot, n_pairs, t);
+      mass_substep_wide<BLOCK, MAXP, WIDE, 0>(smem, p, ms, po, pa, nr_w, live, pslot, pair0, n_pairs, t);
       ++step;
     }
   }
   for (; WIDE == 0 && step + 1 < p.n_steps; step += 2) {
-    mass_substep<SOLVER, BLOCK, MAXP, STRESS, 0>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, n_pairs, t);
+    mass_substep<SOLVER, BLOCK, MAXP, STRESS, 0>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, pair0, n_pairs, t);
     t = t + p.dt;
-    mass_substep<SOLVER, BLOCK, MAXP, STRESS, 1>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, n_pairs, t);
+    mass_substep<SOLVER, BLOCK, MAXP, STRESS, 1>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, pair0, n_pairs, t);
     t = t + p.dt;
   }
   if (WIDE == 0 && step < p.n_steps)
-    mass_substep<SOLVER, BLOCK, MAXP, STRESS, 0>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, n_pairs, t);
+    mass_substep<SOLVER, BLOCK, MAXP, STRESS, 0>(smem, p, ms, rr, st, first, nr, nr_w, live, pslot, pair0, n_pairs, t);
 
   if (live) {
     const uint32_t gi = d.mass_begin + mass;
@@ -1296,8 +1324,11 @@ __device__ __forceinline__ bool position_in_div_range(float4 q) {
 // flags (one per substep parity) record whether any position written for
 // that substep left the fast division's range.
 // WIDE: two records and four entries at a time, the next ones' LDS reads
-// ahead of the arithmetic, for packs of at most kWideMaxMasses masses.
-template <int SOLVER, int BLOCK, int MAXP, bool STRESS, bool WIDE>
+// ahead of the arithmetic, for packs of at most kWideMaxMasses masses.  LAST:
+// the pairs on the last lanes, for packs whose last waves have few records
+// (one order each, known at compile time: chosen per pack in the kernel, with
+// the lane's pair in a register, the loop lost its decoded records and 3-5 %).
+template <int SOLVER, int BLOCK, int MAXP, bool STRESS, bool WIDE, bool LAST = WIDE>
 __global__ __launch_bounds__(BLOCK) void step_massg(StepParams p) {
   static_assert(SOLVER == MH_SOLVER_XPBD_REF,
                 "step_massg stores 12-byte terms: the xpbd step only (the force step_mass is faster)");
@@ -1365,6 +1396,7 @@ __global__ __launch_bounds__(BLOCK) void step_massg(StepParams p) {
     if (live && !position_in_div_range(lds_position<SOLVER>(ms))) atomicOr(&s_flag[0], 1u);
   }
   __syncthreads();
+  const int pair0 = LAST ? BLOCK - 1 - tid : tid;
 
   for (int step = 0; step < p.n_steps; ++step) {
     const float4 own = live ? pos[pslot] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1483,7 +1515,7 @@ __global__ __launch_bounds__(BLOCK) void step_massg(StepParams p) {
       pos[pslot] = np4;
       if (SOLVER == MH_SOLVER_XPBD_REF && !position_in_div_range(np4)) atomicOr(&s_flag[(step + 1) & 1], 1u);
     }
-    mass_pairs_advance<BLOCK, 4>(smem, n_pairs, kDyn, kCst, t + p.dt);
+    mass_pairs_advance<BLOCK, 4>(smem, pair0, n_pairs, kDyn, kCst, t + p.dt);
     t = t + p.dt;
     __syncthreads();
   }
@@ -1565,6 +1597,18 @@ const void* wide_massg() {
   else
     return nullptr;
 }
+// step_massg with the pairs on the last lanes, likewise.  MI355X, us per
+// untracked substep, on the last lanes and on the first: 600 voxel robots of
+// 216 masses 4.26 and 4.33, of 729 13.61 and 13.63 (tracked 15.5 and 15.8);
+// lists of equal length (760 masses, 600 robots), 2 springs each 4.84 and
+// 4.57, 6 springs 6.79 and 6.28, 26 springs 15.2 and 14.5.
+template <int SOLVER, int BLOCK, int MAXP, bool STRESS>
+const void* uneven_massg() {
+  if constexpr (BLOCK == 768)
+    return reinterpret_cast<const void*>(&step_massg<SOLVER, BLOCK, MAXP, STRESS, false, true>);
+  else
+    return nullptr;
+}
 
 #define MH_MASS(SOLVER, B, P)                                                         \
   {SOLVER, MH_KERNEL_MASS, 0, B, P, 1, reinterpret_cast<const void*>(&step_mass<SOLVER, B, P, false>), \
@@ -1573,7 +1617,8 @@ const void* wide_massg() {
 #define MH_MASSG(SOLVER, B, P)                                                        \
   {SOLVER, MH_KERNEL_MASS, 1, B, P, 1, reinterpret_cast<const void*>(&step_massg<SOLVER, B, P, false, false>), \
    reinterpret_cast<const void*>(&step_massg<SOLVER, B, P, (SOLVER == MH_SOLVER_XPBD_REF), false>), \
-   wide_massg<SOLVER, B, P, false>(), wide_massg<SOLVER, B, P, true>()}
+   wide_massg<SOLVER, B, P, false>(), wide_massg<SOLVER, B, P, true>(),                 \
+   uneven_massg<SOLVER, B, P, false>(), uneven_massg<SOLVER, B, P, true>()}
 #define MH_CHUNK(SOLVER, B, M) \
   {SOLVER, MH_KERNEL_STREAM, 1, B, 0, M, reinterpret_cast<const void*>(&step_chunk<SOLVER, B, M>)}
 #define MH_STREAM(SOLVER, B) \
@@ -1648,19 +1693,19 @@ size_t lds_bytes_stream(int mass_cap, int n_mat) {
   return 16u * static_cast<size_t>(mass_cap) + 4u * static_cast<size_t>(n_mat);
 }
 
-hipError_t launch_step(const KernelVariant& v, int n_packs, size_t lds_bytes, int compute_units, hipStream_t stream,
-                       const StepParams& p) {
+hipError_t launch_step(const KernelVariant& v, const LaunchShape& l, hipStream_t stream, const StepParams& p) {
   StepParams args = p;
   void* kargs[] = {&args};
   const void* fn = (p.track_stress && v.fn_stress) ? v.fn_stress : v.fn;
   if (v.kind == MH_KERNEL_MASS && v.chunked == 1) {
     if (v.fn_wide && p.mass_cap <= kWideMaxMasses) fn = p.track_stress ? v.fn_wide_stress : v.fn_wide;
-  } else if (v.fn_wide && n_packs <= compute_units) {
+    else if (v.fn_uneven && l.uneven) fn = p.track_stress ? v.fn_uneven_stress : v.fn_uneven;
+  } else if (v.fn_wide && l.n_packs <= l.compute_units) {
     fn = v.fn_wide;
   }
   // the mass-parallel streaming kernel's LDS is a static array
-  const size_t dyn = (v.kind == MH_KERNEL_STREAM && v.chunked == 2) ? 0 : lds_bytes;
-  return hipLaunchKernel(fn, dim3(n_packs), dim3(v.block), kargs, dyn, stream);
+  const size_t dyn = (v.kind == MH_KERNEL_STREAM && v.chunked == 2) ? 0 : l.lds_bytes;
+  return hipLaunchKernel(fn, dim3(l.n_packs), dim3(v.block), kargs, dyn, stream);
 }
 
 hipError_t launch_clock(float* times, float t0, float dt, int n_steps, int K, hipStream_t stream) {
