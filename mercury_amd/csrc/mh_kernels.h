@@ -90,7 +90,11 @@ struct LaunchShape {
   int n_packs;
   size_t lds_bytes;
   int compute_units;
-  bool uneven;  // mass-parallel: in most packs the last wave with masses has at most half the first's records
+  // mass-parallel parts: in most packs the last wave with masses has at most
+  // half the first's records; most records (step_massg: springs from their
+  // first endpoint) of one mass
+  bool uneven;
+  int longest;
 };
 
 // All compiled variants (table lives in step_kernels.hip).

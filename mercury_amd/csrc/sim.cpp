@@ -98,7 +98,8 @@ struct Part {
   size_t lds = 0;
   uint32_t pack_offset = 0;         // first descriptor in the device array
   int n_robots = 0;
-  bool uneven = false;              // LaunchShape::uneven
+  bool uneven = false;              // LaunchShape's
+  int longest = 0;
 };
 
 // Robots that fit the LDS kernel go to the LDS part, the rest to the
@@ -643,6 +644,7 @@ void upload_mass(mh_sim* s, Part& part, std::vector<uint16_t>& perm, std::vector
   mcnt.resize(cnt_end);
   // pass 2 (packs in parallel): pairs, lane order and records
   std::atomic<size_t> n_uneven{0};
+  std::vector<uint8_t> pack_longest(n_packs, 0);
   parallel_for(n_packs, [&](size_t pi) {
     const PackDesc& d = part.packs[pi];
     const std::vector<uint64_t>& table = tables[pi];
@@ -745,8 +747,10 @@ void upload_mass(mh_sim* s, Part& part, std::vector<uint16_t>& perm, std::vector
       return n;
     };
     if (nm && 2 * longest((nm - 1) & ~63u, nm) <= longest(0, std::min(nm, 64u))) n_uneven++;
+    pack_longest[pi] = longest(0, nm);
   });
   part.uneven = 2 * n_uneven > n_packs;
+  for (uint8_t n : pack_longest) part.longest = std::max<int>(part.longest, n);
   std::stable_sort(part.packs.begin(), part.packs.end(), [](const PackDesc& x, const PackDesc& y) {
     return static_cast<uint64_t>(x.n_spring) + x.n_mass > static_cast<uint64_t>(y.n_spring) + y.n_mass;
   });
@@ -975,7 +979,7 @@ int issue(mh_sim* s, int n_steps, int track) {
     for (int done = 0; done < n_steps;) {
       const int n = std::min(K, n_steps - done);
       StepParams p = make_params(s, part, launches, n, track);
-      const LaunchShape shape{static_cast<int>(part.packs.size()), part.lds, s->compute_units, part.uneven};
+      const LaunchShape shape{static_cast<int>(part.packs.size()), part.lds, s->compute_units, part.uneven, part.longest};
       hip_check(launch_step(*part.v, shape, st, p), "step launch");
       done += n;
       launches++;

@@ -1214,8 +1214,15 @@ __global__ __launch_bounds__(BLOCK) void step_mass(StepParams p) {
 // batches cost 1-4 %.  MI355X, ms per 1000 untracked substeps, plain and
 // wide: one robot of 125 masses 3.79 and 2.84, of 343 3.88 and 3.20, of 512
 // 4.03 and 3.76, of 729 4.48 and 4.65; 512 robots of 512 masses 8.21 and
-// 7.84, of 686 masses per pack 4.48 and 4.62, of 729 9.15 and 9.50.
+// 7.84, of 686 masses per pack 4.48 and 4.62, of 729 9.15 and 9.50.  Lists of
+// one record leave half of every batch unused, which more than 256 masses do
+// not hide: 600 robots of 256 masses 3.73 and 3.50, of 257 3.95 and 4.07, of
+// 512 4.04 and 4.15 (tracked; 2 records 512 masses 4.56 and 4.02, 3 records
+// 5.77 and 5.65).
 constexpr int kWideMaxMasses = 512;
+inline bool massg_wide(int masses, int longest) {
+  return masses <= 256 || (masses <= kWideMaxMasses && longest != 1);
+}
 
 // XPBD term of the gather kernel.  fast_ok says that the workgroup's
 // positions and the pack's materials lie where div_rn_from_rcp is exact
@@ -1698,7 +1705,7 @@ hipError_t launch_step(const KernelVariant& v, const LaunchShape& l, hipStream_t
   void* kargs[] = {&args};
   const void* fn = (p.track_stress && v.fn_stress) ? v.fn_stress : v.fn;
   if (v.kind == MH_KERNEL_MASS && v.chunked == 1) {
-    if (v.fn_wide && p.mass_cap <= kWideMaxMasses) fn = p.track_stress ? v.fn_wide_stress : v.fn_wide;
+    if (v.fn_wide && massg_wide(p.mass_cap, l.longest)) fn = p.track_stress ? v.fn_wide_stress : v.fn_wide;
     else if (v.fn_uneven && l.uneven) fn = p.track_stress ? v.fn_uneven_stress : v.fn_uneven;
   } else if (v.fn_wide && l.n_packs <= l.compute_units) {
     fn = v.fn_wide;

@@ -24,19 +24,25 @@ def ring(n, reach, pairs):
     return e
 
 
-@pytest.mark.parametrize("solver,stress", [("force", False), ("xpbd", False), ("xpbd", True)])
-@pytest.mark.parametrize("shape,block", [((760, 3, 30), 768), ((600, 1, 2), 768), ((700, 8, 480), 768),
-                                         ((250, 2, 500), 256), ((1000, 2, 40), 1024), ((512, 3, 200), 512),
-                                         ("voxels", 768), ("voxels", 256)], ids=str)
+CASES = [(shape, block, solver, stress)
+         for shape, block in (((760, 3, 30), 768), ((600, 1, 2), 768), ((700, 8, 480), 768), ((250, 2, 500), 256),
+                              ((1000, 2, 40), 1024), ((512, 3, 200), 512), ("voxels", 768), ("voxels", 256))
+         for solver, stress in (("force", False), ("xpbd", False), ("xpbd", True), ("gather", False), ("gather", True))
+         if solver != "gather" or block < 1024]  # the gather kernel's blocks
+
+
+@pytest.mark.parametrize("shape,block,solver,stress", CASES, ids=str)
 def test_pair_order_exact(shape, block, solver, stress):
     print("pair order", shape, block, solver, stress, flush=True)
     if shape == "voxels":
         case = workload_case(n_robots=3, voxels=8 if block == 768 else 5, seed=2)
     else:
         case = Case([ring(*shape)] * 2, mh.workload_materials(), mh.materials.WORKLOAD_ROWS)
-    so = mh.MH_SOLVER_XPBD_REF if solver == "xpbd" else mh.MH_SOLVER_FORCE
+    so = mh.MH_SOLVER_FORCE if solver == "force" else mh.MH_SOLVER_XPBD_REF
     env = LAND if solver == "force" else None
-    sim = gpu_sim(case, so, 1e-4, env, kernel=mh.MH_KERNEL_MASS, block_size=block, robots_per_block=1)
+    kernel = mh.MH_KERNEL_MASS_GATHER if solver == "gather" else mh.MH_KERNEL_MASS
+    sim = gpu_sim(case, so, 1e-4, env, kernel=kernel, block_size=block, robots_per_block=1)
+    assert sim.info().kernel == kernel and sim.info().block_size == block
     sim.Step(61, trackStresses=stress)
     want = mirror(case, so, 61, 1e-4, env, stress=stress)
     assert np.abs(want[1]).max() > 0
