@@ -2,11 +2,11 @@
 //
 // Replaces Triangulation::KNN (common/evolvables/knn.cu:62-144: dense M x M
 // distance matrix + segmented radix sort per row).  Robots of up to 2048
-// masses, from 6 neighbours on: one wave per query, the robot's positions in
-// the wave's registers; otherwise one lane per query, a scan over LDS tiles.  Distances are
-// sqrtf(dx*dx + (dy*dy + dz*dz)) (Eigen's Vector3f::norm order, as KNN_CPU
-// computes them, knn.cu:147-158); a zero distance -- the mass itself or a
-// coincident mass -- counts as +inf
+// masses, from 6 neighbours on (16 under 64 masses): one wave per query, the
+// robot's positions in the wave's registers; otherwise one lane per query, a
+// scan over LDS tiles.  Distances are sqrtf(dx*dx + (dy*dy + dz*dz)) (Eigen's
+// Vector3f::norm order, as KNN_CPU computes them, knn.cu:147-158); a zero
+// distance -- the mass itself or a coincident mass -- counts as +inf
 // (knn.cu:166-167); equal distances keep the lower index first, the order
 // the reference's stable radix sort of index-ordered rows produces.
 #include <hip/hip_runtime.h>
@@ -114,23 +114,32 @@ __global__ __launch_bounds__(kQueryBlock) void knn_tiles(const float* __restrict
 // candidates lie at one distance, the distances below that one D and the
 // lowest indices at it are taken.
 //
-// What bounds it: VALU issue (per query 8 instructions for each 64 squared
+// What bounds it: VALU issue (per query 10 instructions for each 64 squared
 // distances and 2 per try of T, then the ranking).  The scan spends its time
 // on insertions: nearly every candidate enters the list of some lane of the
 // wave, and an entry moves K pairs.  MI355X, K = 25, 384 robots of 200 to
 // 2000 masses: the kernels 5.53 -> 0.99 ms, the call 11.6 -> 7.1 (the rest is
 // allocations and copies of the results).  One robot of 2000 masses 3.3 ->
-// 0.15 ms.  Slower than the scan: clouds with two distinct points only, at
-// few neighbours (1100 masses, K = 6: 718 and 972 us).
+// 0.15 ms.  Clouds of few distinct points have few insertions, which the scan
+// is fast at, and no threshold admits 64 of them; nearest_levels serves them
+// (kernel, us, scan / this one, K = 6: 128 robots of 1100 masses at two points
+// 185 / 151, 200 of 300 60 / 30; without it 437 and 62).  Still slower than
+// the scan: robots of about 100 masses or fewer at few points (100 robots of
+// 64 masses at two points, K = 6, 17 / 34), and some clouds of many scales (128
+// of 1100 masses over 12 decades, K = 6, 523 / 572).
 //   kWaveQueries: 64 queries per wave left small robots on too few waves
 //     (the robots of at most 512 masses 219 us, at 16 per wave 55).
 //   kWaveMinK: a short list is cheap to insert into: 128 robots of 1100
-//     masses on a lattice, scan and this kernel: K = 2 597 and 700 us, 4 832
-//     and 853, 6 1078 and 973, 12 1743 and 1361.
-//   kWaveMaxMasses: 32 candidates a lane take 219 VGPRs, two waves per SIMD.
+//     masses on a lattice, K = 6 1078 us by the scan and 973 by this kernel,
+//     12 1743 and 1361.  Under kWaveSmall masses the wave is not full: calls
+//     of 300 robots of 40 masses, K = 8, 119 and 123 us uniform, 98 and 109 all
+//     at one point, K = 12 139 and 137, 111 and 123, K = 16 159 and 152.
+//   kWaveMaxMasses: 32 candidates a lane take 221 VGPRs, two waves per SIMD.
 constexpr int kWaveQueries = 16;  // per wave
 constexpr int kWaveMaxMasses = 2048;
 constexpr int kWaveMinK = 6;
+constexpr uint32_t kWaveSmall = 64;
+constexpr int kWaveMinKSmall = 16;
 static_assert(kMaxK < 64, "admitted candidates fit a wave");
 
 // orders a wave's own LDS accesses
@@ -163,6 +172,41 @@ __device__ __forceinline__ int wave_rank(float2* kept, int lane, int c, float d,
   return rank;
 }
 
+// Clouds of few distinct points: the K nearest of the candidates s (squared
+// distances, NaN: none) by one level of distance after the other, each in
+// index order, into kept -- in rank order, nothing is left to sort.  False
+// where three levels hold fewer than K (kept is then undefined).
+template <int NC>
+__device__ __forceinline__ bool nearest_levels(const float (&s)[NC], float2* kept, int lane, int K) {
+  int base = 0;
+  float after = 0.0f;  // squared distances up to here are in kept
+  for (int level = 0; level < 3; ++level) {
+    float m = INFINITY;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) m = s[i] > after ? fminf(m, s[i]) : m;
+    for (int off = 32; off > 0; off >>= 1) m = fminf(m, __shfl_xor(m, off));
+    m = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(m)));
+    if (m == INFINITY) break;
+    // the floats from m up with its root, one a lane
+    const uint64_t roots = __builtin_amdgcn_ballot_w64(sqrtf(__uint_as_float(__float_as_uint(m) + lane)) == sqrtf(m));
+    after = __uint_as_float(__float_as_uint(m) + 63 - __builtin_clzll(roots));
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      if (base >= K) break;
+      const bool in = s[i] >= m && s[i] <= after;
+      const uint64_t lanes = __builtin_amdgcn_ballot_w64(in);
+      const int at = base + lanes_below(lanes);
+      if (in && at < K) kept[at] = make_float2(s[i], __int_as_float(lane + 64 * i));
+      base += __popcll(lanes);
+    }
+    if (base >= K) {
+      wave_sync();
+      return true;
+    }
+  }
+  return false;
+}
+
 template <int NC>
 __global__ __launch_bounds__(256, 2) void knn_waves(const float* __restrict__ pos, const KnnTile* __restrict__ tiles,
                                                     int K, uint16_t* __restrict__ nbr, float* __restrict__ dist) {
@@ -185,6 +229,7 @@ __global__ __launch_bounds__(256, 2) void knn_waves(const float* __restrict__ po
   const int q_end = min(n, q0 + kWaveQueries);
   constexpr float kMax = 3.402823466e+38f;
   float T = 1.0f;  // threshold on the squared distance, 0 < T <= kMax
+  bool tied = false;  // the last query had more than 64 candidates at one distance
   for (int q = q0; q < q_end; ++q) {
     const float qx = p[3 * q], qy = p[3 * q + 1], qz = p[3 * q + 2];
     // squared distances; NaN, which passes no comparison, for what is no
@@ -197,6 +242,16 @@ __global__ __launch_bounds__(256, 2) void knn_waves(const float* __restrict__ po
       s[i] = v > 0.0f ? v : __builtin_nanf("");
     }
     const size_t o = (static_cast<size_t>(t.out_begin) + q) * K;
+    if (tied && nearest_levels<NC>(s, kept, lane, K)) {
+      if (lane < K) {
+        const float2 e = kept[lane];
+        nbr[o + lane] = static_cast<uint16_t>(__float_as_int(e.y));
+        dist[o + lane] = sqrtf(e.x);
+      }
+      wave_sync();
+      continue;
+    }
+    tied = false;
     // lo admits too few, hi too many (bit patterns of positive floats order
     // as they do).  Every try lies strictly between and becomes one of them,
     // so the search ends.
@@ -262,6 +317,7 @@ __global__ __launch_bounds__(256, 2) void knn_waves(const float* __restrict__ po
       if (hi - lo <= 1u) {  // all between lo and hi lie at sqrtf(hi)
         T = __uint_as_float(hi);
         D = sqrtf(T);
+        tied = true;
         break;
       }
       if (top) {  // and one float below it: many candidates may lie there
@@ -309,6 +365,7 @@ __global__ __launch_bounds__(256, 2) void knn_waves(const float* __restrict__ po
       nbr[o + rank] = static_cast<uint16_t>(idx);
       dist[o + rank] = d;
     }
+    T = fminf(T * 1.0001f, kMax);  // past this distance, which the next query may share
   }
 }
 
@@ -335,7 +392,7 @@ int mh_knn_batch(int device, int n_robots, const uint32_t* mass_offset, const fl
     if (mass_offset[r + 1] < mass_offset[r]) return fail(MH_ERR_ARG, "offsets must be non-decreasing");
     if (m > 65535) return fail(MH_ERR_RANGE, "robot has more than 65535 masses");
     if (m > 0 && static_cast<int>(m) <= K) return fail(MH_ERR_RANGE, "robot has no more than K masses");
-    const bool scan = m > kWaveMaxMasses || K < kWaveMinK;
+    const bool scan = m > kWaveMaxMasses || K < (m < kWaveSmall ? kWaveMinKSmall : kWaveMinK);
     std::vector<KnnTile>& kind = kinds[scan ? 4 : m <= 512 ? 0 : (m - 1) / 512];
     const uint32_t block = scan ? kQueryBlock : 4 * kWaveQueries;
     for (uint32_t q = 0; q < m; q += block) kind.push_back({mass_offset[r], m, q, mass_offset[r]});
