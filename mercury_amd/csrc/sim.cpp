@@ -151,7 +151,8 @@ struct mh_sim {
   // device state
   mh::DevBuf<float4> pos, vel;
   mh::DevBuf<float> lbar, stress, scratch, com;
-  mh::DevBuf<float> xyz;          // packed positions or velocities (mh_sim_collect)
+  mh::DevBuf<float> xyz;          // packed positions or velocities (mh_sim_collect); kept from one population
+                                  // to the next of at least half its masses
   bool stress_zero = true;        // nothing has written the stress buffer since it was cleared
   mh::DevBuf<uint8_t> smat, mass_id;
   mh::DevBuf<uint16_t> mperm, ccsr, crow;
@@ -1329,7 +1330,7 @@ int mh_sim_set_population(mh_sim* s, const mh_population* pop) {
   s->stress.alloc(std::max<size_t>(s->n_active, 1));
   mh::hip_check(hipMemsetAsync(s->stress.p, 0, sizeof(float) * s->stress.n, s->stream), "memset");
   s->stress_zero = true;
-  s->xyz.release();
+  if (s->xyz.n > 6 * M) s->xyz.release();
   s->com.alloc(3 * std::max(R, 1));
   mh::upload_materials(s);
   if (R > 0) mh::choose_plan(s);
@@ -1460,7 +1461,7 @@ int mh_sim_set_voxel_population(mh_sim* s, int n_robots, int nx, int ny, int nz,
   s->stress.alloc(std::max<size_t>(ST, 1));
   mh::hip_check(hipMemsetAsync(s->stress.p, 0, sizeof(float) * s->stress.n, s->stream), "memset");
   s->stress_zero = true;
-  s->xyz.release();
+  if (s->xyz.n > 6 * M) s->xyz.release();
   s->com.alloc(3 * std::max(R, 1));
   s->vox_enc.alloc(M);
   if (M)
@@ -1652,13 +1653,32 @@ int mh_sim_collect(mh_sim* s, float* pos, float* vel, float* stress) {
   const size_t M = s->n_masses;
   mh::hip_check(hipSetDevice(s->cfg.device), "hipSetDevice");
   // packed on the device and copied straight into the caller's arrays
-  // (406000 masses: 0.63 -> 0.35 ms each against repacking on the host)
-  if ((pos || vel) && M && s->xyz.n < 3 * M) s->xyz.alloc(3 * M);
+  // (406000 masses: 0.63 -> 0.35 ms each against repacking on the host, which
+  // a full device leaves)
+  if ((pos || vel) && M && s->xyz.n < 3 * M) {
+    try {
+      s->xyz.alloc(3 * M);
+    } catch (const mh::Error&) {
+      (void)hipGetLastError();
+    }
+  }
+  std::vector<float4> host;
   auto fetch = [&](const float4* src, float* out) {
     if (!out || !M) return;
-    mh::hip_check(mh::launch_xyz(src, s->xyz.p, M, s->stream), "pack launch");
-    mh::hip_check(hipMemcpyAsync(out, s->xyz.p, 3 * M * sizeof(float), hipMemcpyDeviceToHost, s->stream), "D2H");
+    if (s->xyz.n >= 3 * M) {
+      mh::hip_check(mh::launch_xyz(src, s->xyz.p, M, s->stream), "pack launch");
+      mh::hip_check(hipMemcpyAsync(out, s->xyz.p, 3 * M * sizeof(float), hipMemcpyDeviceToHost, s->stream), "D2H");
+      mh::hip_check(hipStreamSynchronize(s->stream), "D2H");
+      return;
+    }
+    host.resize(M);
+    mh::hip_check(hipMemcpyAsync(host.data(), src, M * sizeof(float4), hipMemcpyDeviceToHost, s->stream), "D2H");
     mh::hip_check(hipStreamSynchronize(s->stream), "D2H");
+    for (size_t i = 0; i < M; i++) {
+      out[3 * i] = host[i].x;
+      out[3 * i + 1] = host[i].y;
+      out[3 * i + 2] = host[i].z;
+    }
   };
   fetch(s->pos.p, pos);
   fetch(s->vel.p, vel);
