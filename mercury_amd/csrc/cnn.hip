@@ -992,11 +992,10 @@ void loss_backward_to(mh_cnn* net, const uint8_t* genomes, const float* target, 
 
 // The packed weights of every layer from the fp32 parameters.
 void refresh_weights(mh_cnn* net) {
-  for (int l = 0; l < kNL; l++) {
-    const PackedLayer& p = l < 3 ? net->conv[l] : net->head.layer[l - 3];
-    hipLaunchKernelGGL(pack_layer, dim3(blocks_for(static_cast<size_t>(p.out) * p.in)), dim3(256), 0, net->stream, p,
-                       net->params.p, net->pack.p, static_cast<uint16_t*>(nullptr));
-  }
+  PackList list{kNL, {}};
+  static_assert(kNL <= kPackLayers, "every layer in one launch");
+  for (int l = 0; l < kNL; l++) list.layer[l] = l < 3 ? net->conv[l] : net->head.layer[l - 3];
+  launch_pack(list, net->params.p, net->pack.p, nullptr, net->stream);
   hipcheck(hipGetLastError(), "weights");
 }
 

@@ -69,12 +69,32 @@ __device__ __forceinline__ void pack_store(const PackedLayer& p, uint16_t* pack,
   pack[p.bwd + packed_index(k * p.out + o, c, (p.c + 15) >> 4)] = b;
 }
 
-// plain (may be null): the bf16 weights as they lie in the parameter vector
-__global__ void pack_layer(PackedLayer p, const float* params, uint16_t* pack, uint16_t* plain) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= p.out * p.in) return;
-  pack_store(p, pack, e / p.in, e % p.in, params[p.w_off + e]);
-  if (plain) plain[p.w_off + e] = weight_bits(params[p.w_off + e]);
+// The packings of every layer of a network from its fp32 parameters.  plain
+// (may be null): the bf16 weights as they lie in the parameter vector.
+constexpr int kPackLayers = 6;
+struct PackList {
+  int n;
+  PackedLayer layer[kPackLayers];
+};
+__global__ void pack_layers(PackList list, const float* params, uint16_t* pack, uint16_t* plain) {
+  int e = blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+  for (int l = 0; l < kPackLayers; ++l) {
+    if (l >= list.n) return;
+    const PackedLayer& p = list.layer[l];
+    if (e < p.out * p.in) {
+      const float w = params[p.w_off + e];
+      pack_store(p, pack, e / p.in, e % p.in, w);
+      if (plain) plain[p.w_off + e] = weight_bits(w);
+      return;
+    }
+    e -= p.out * p.in;
+  }
+}
+inline void launch_pack(const PackList& list, const float* params, uint16_t* pack, uint16_t* plain, hipStream_t s) {
+  int n = 0;
+  for (int l = 0; l < list.n; l++) n += list.layer[l].out * list.layer[l].in;
+  hipLaunchKernelGGL(pack_layers, dim3((n + 255) / 256), dim3(256), 0, s, list, params, pack, plain);
 }
 
 __global__ void fill_zero_u16(uint16_t* p, int n) {

@@ -118,11 +118,9 @@ void ensure_batch(mh_mlp* net, int B) {
 // fp32 parameters.
 void refresh_weights(mh_mlp* net) {
   if (net->fused) {
-    for (int l = 0; l < net->L(); l++) {
-      const PackedLayer& p = net->shape.layer[l];
-      hipLaunchKernelGGL(pack_layer, dim3((p.out * p.in + 255) / 256), dim3(256), 0, net->stream, p, net->params.p,
-                         net->pack.p, reinterpret_cast<uint16_t*>(net->w16.p));
-    }
+    PackList list{net->L(), {}};
+    std::copy_n(net->shape.layer, net->L(), list.layer);
+    launch_pack(list, net->params.p, net->pack.p, reinterpret_cast<uint16_t*>(net->w16.p), net->stream);
   } else {
     hipLaunchKernelGGL(to_bf16, dim3((net->n_params + 255) / 256), dim3(256), 0, net->stream, net->params.p,
                        net->w16.p, static_cast<int>(net->n_params));
