@@ -880,7 +880,7 @@ struct LayerShape {
   int out, in;  // weight [out x in], bias [out]
 };
 constexpr LayerShape kLayers[] = {{kC1, kK1}, {kC2, kK2}, {kC3, kK3}, {kH, kC3}, {kH, kH}, {1, kH}};
-constexpr int kNL = 6;
+constexpr int kNL = 6, kHeadL = 3;
 
 }  // namespace
 
@@ -945,12 +945,12 @@ ConvNet conv_net(const mh_cnn* net, const uint8_t* genomes, const int* idx) {
   return ConvNet{net->conv[0], net->conv[1], net->conv[2], net->params.p, net->pack.p, genomes, idx};
 }
 
-// y [B] of the genomes on the device
+// y [B] of the genomes on the device (chunks of up to 4096: 16-row tiles in
+// the head, as mh_mlp_forward's)
 void forward(mh_cnn* net, const uint8_t* genomes, int B, float* feat, float* y) {
   hipLaunchKernelGGL((conv_features<false>), dim3(B), dim3(512), 0, net->stream, conv_net(net, genomes, nullptr), feat,
                      ConvTrain{});
-  if (B <= 4096) launch_dense_net<1, false>(net->head, net->params.p, net->pack.p, feat, B, y, DenseTrain{}, net->stream);
-  else launch_dense_net<2, false>(net->head, net->params.p, net->pack.p, feat, B, y, DenseTrain{}, net->stream);
+  launch_dense_net_of<kHeadL, 1, false>(net->head, net->params.p, net->pack.p, feat, B, y, DenseTrain{}, net->stream);
   hipcheck(hipGetLastError(), "cnn forward");
 }
 
@@ -975,11 +975,11 @@ void loss_backward_to(mh_cnn* net, const uint8_t* genomes, const float* target, 
     tr.D[l] = net->hd[l].p;
     tr.delta[l] = net->hdelta[l].p;
   }
-  launch_dense_net<1, true>(net->head, net->params.p, net->pack.p, net->feat.p, B, nullptr, tr, s);
+  launch_dense_net_of<kHeadL, 1, true>(net->head, net->params.p, net->pack.p, net->feat.p, B, nullptr, tr, s);
   hipLaunchKernelGGL(conv_backward, dim3(B), dim3(512), 0, s, cn, ct);
   const AdamArgs ad = adam ? *adam : AdamArgs{};
-  if (adam) launch_dense_wgrad<1, 8, true>(net->head, tr, ad, nullptr, s);
-  else launch_dense_wgrad<1, 8, false>(net->head, tr, ad, net->grads.p, s);
+  if (adam) launch_dense_wgrad_of<kHeadL, 1, 8, true>(net->head, tr, ad, nullptr, s);
+  else launch_dense_wgrad_of<kHeadL, 1, 8, false>(net->head, tr, ad, net->grads.p, s);
   hipLaunchKernelGGL(conv_wgrad, dim3(kSplit, kRoles), dim3(512), 0, s, cn, ct, B, net->part.p, net->n_conv);
   const int n = static_cast<int>(net->n_conv);
   if (adam)
@@ -1039,7 +1039,7 @@ int mh_cnn_create(int device, uint64_t seed, mh_cnn** out) {
     }
     net->n_params = off;
     net->n_conv = net->w_off[3];
-    net->head.L = 3;
+    net->head.L = kHeadL;
     net->head.zero = at;
     at += 8;
     // He-uniform weights (bound sqrt(6 / fan_in)), zero biases

@@ -72,6 +72,7 @@ __device__ __forceinline__ void pack_store(const PackedLayer& p, uint16_t* pack,
 // The packings of every layer of a network from its fp32 parameters.  plain
 // (may be null): the bf16 weights as they lie in the parameter vector.
 constexpr int kPackLayers = 6;
+static_assert(kDenseMaxLayers <= kPackLayers, "a fused network packs in one launch");
 struct PackList {
   int n;
   PackedLayer layer[kPackLayers];
@@ -119,9 +120,6 @@ struct RowSplits {
 inline RowSplits row_splits(int B, int splits) {
   const int rows = (B + splits - 1) / splits;
   return RowSplits{B, splits, rows, (rows + 31) / 32};
-}
-inline size_t operand_elements(const RowSplits& r, int n) {
-  return static_cast<size_t>(r.splits) * r.slices * ((n + 15) / 16) * 512;
 }
 // Where rows row .. row + 3 (row a multiple of 4) of such an operand lie:
 // element (row + r, 16 t + c) at slice(r) * tiles * 512 + t * 512 + c * 8 +
@@ -621,29 +619,39 @@ __global__ __launch_bounds__(kWgThreads) void dense_wgrad(DenseShape sh, DenseTr
   }
 }
 
-// dense_net and dense_wgrad for the network's layer count.
+// dense_net and dense_wgrad of a network of L layers, and for any layer count.
+template <int L, int MT, bool TRAIN>
+void launch_dense_net_of(const DenseShape& sh, const float* params, const uint16_t* pack, const float* x, int B,
+                         float* y, const DenseTrain& tr, hipStream_t s) {
+  hipLaunchKernelGGL((dense_net<L, MT, TRAIN>), dim3((B + 16 * MT - 1) / (16 * MT)), dim3(kDenseThreads), 0, s, sh,
+                     params, pack, x, B, y, tr);
+  hipcheck(hipGetLastError(), "dense layers");
+}
+template <int L, int JT, int SR, bool ADAM>
+void launch_dense_wgrad_of(const DenseShape& sh, const DenseTrain& tr, const AdamArgs& ad, float* grads,
+                           hipStream_t s) {
+  hipLaunchKernelGGL((dense_wgrad<L, JT, SR, ADAM>), dim3(dense_wgrad_blocks(sh, JT)), dim3(kWgThreads), 0, s, sh, tr,
+                     ad, grads);
+  hipcheck(hipGetLastError(), "dense weight gradients");
+}
 template <int MT, bool TRAIN>
 void launch_dense_net(const DenseShape& sh, const float* params, const uint16_t* pack, const float* x, int B, float* y,
                       const DenseTrain& tr, hipStream_t s) {
-  const dim3 grid((B + 16 * MT - 1) / (16 * MT));
   switch (sh.L) {
-    case 1: hipLaunchKernelGGL((dense_net<1, MT, TRAIN>), grid, dim3(kDenseThreads), 0, s, sh, params, pack, x, B, y, tr); break;
-    case 2: hipLaunchKernelGGL((dense_net<2, MT, TRAIN>), grid, dim3(kDenseThreads), 0, s, sh, params, pack, x, B, y, tr); break;
-    case 3: hipLaunchKernelGGL((dense_net<3, MT, TRAIN>), grid, dim3(kDenseThreads), 0, s, sh, params, pack, x, B, y, tr); break;
-    default: hipLaunchKernelGGL((dense_net<4, MT, TRAIN>), grid, dim3(kDenseThreads), 0, s, sh, params, pack, x, B, y, tr);
+    case 1: return launch_dense_net_of<1, MT, TRAIN>(sh, params, pack, x, B, y, tr, s);
+    case 2: return launch_dense_net_of<2, MT, TRAIN>(sh, params, pack, x, B, y, tr, s);
+    case 3: return launch_dense_net_of<3, MT, TRAIN>(sh, params, pack, x, B, y, tr, s);
+    default: launch_dense_net_of<4, MT, TRAIN>(sh, params, pack, x, B, y, tr, s);
   }
-  hipcheck(hipGetLastError(), "dense layers");
 }
 template <int JT, int SR, bool ADAM>
 void launch_dense_wgrad(const DenseShape& sh, const DenseTrain& tr, const AdamArgs& ad, float* grads, hipStream_t s) {
-  const dim3 grid(dense_wgrad_blocks(sh, JT)), block(kWgThreads);
   switch (sh.L) {
-    case 1: hipLaunchKernelGGL((dense_wgrad<1, JT, SR, ADAM>), grid, block, 0, s, sh, tr, ad, grads); break;
-    case 2: hipLaunchKernelGGL((dense_wgrad<2, JT, SR, ADAM>), grid, block, 0, s, sh, tr, ad, grads); break;
-    case 3: hipLaunchKernelGGL((dense_wgrad<3, JT, SR, ADAM>), grid, block, 0, s, sh, tr, ad, grads); break;
-    default: hipLaunchKernelGGL((dense_wgrad<4, JT, SR, ADAM>), grid, block, 0, s, sh, tr, ad, grads);
+    case 1: return launch_dense_wgrad_of<1, JT, SR, ADAM>(sh, tr, ad, grads, s);
+    case 2: return launch_dense_wgrad_of<2, JT, SR, ADAM>(sh, tr, ad, grads, s);
+    case 3: return launch_dense_wgrad_of<3, JT, SR, ADAM>(sh, tr, ad, grads, s);
+    default: launch_dense_wgrad_of<4, JT, SR, ADAM>(sh, tr, ad, grads, s);
   }
-  hipcheck(hipGetLastError(), "dense weight gradients");
 }
 
 }  // namespace
