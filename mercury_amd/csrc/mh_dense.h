@@ -172,7 +172,7 @@ struct DenseTrain {
   uint16_t* X[kDenseMaxLayers];        // input of layer l, as a weight-gradient operand
   uint16_t* D[kDenseMaxLayers];        // loss gradient of layer l's output, likewise
   float* delta[kDenseMaxLayers];       // and in fp32, [B x out], for the bias sums
-  float* dx;                           // gradient of the input, [B x in]; null: not wanted
+  float* dx;                           // gradient of the input, [B x in]; null: not wanted (one layer: has to be)
 };
 
 // Every layer for 16 MT rows per workgroup (8 waves, output tiles w and w + 8
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_net(DenseShape sh, const 
     }
     *reinterpret_cast<u16x8_t*>(&act[0][r][k]) = v;
   }
-  if (kStages > 1) fetch(1, 0, kSlices);
+  if (L > 1) fetch(1, 0, kSlices);
   // operands for the stores at the end: every layer's input and output
   // gradient
   uint2 xo[TRAIN ? L : 1][T], go[TRAIN ? L : 1][T];
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_net(DenseShape sh, const 
   for (int st = 0; st < kStages; ++st) {
     const bool fwd = st < L;
     const int l = fwd ? st : 2 * L - 1 - st;
-    if (TRAIN && st == kStages - 1 && !tr.dx) break;
+    if (TRAIN && st == kStages - 1 && (L == 1 || !tr.dx)) break;
     const int no = fwd ? out_[l] : in_[l];
     const uint16_t (*a)[kActPitch] = act[st & 1];
     uint16_t (*b)[kActPitch] = act[1 - (st & 1)];
@@ -623,6 +623,9 @@ __global__ __launch_bounds__(kWgThreads) void dense_wgrad(DenseShape sh, DenseTr
 template <int L, int MT, bool TRAIN>
 void launch_dense_net_of(const DenseShape& sh, const float* params, const uint16_t* pack, const float* x, int B,
                          float* y, const DenseTrain& tr, hipStream_t s) {
+  // a network of one layer has no stage before the input gradient in which
+  // its weights could be requested
+  if (L == 1 && tr.dx) throw mh::Error(MH_ERR_INTERNAL, "input gradient of a one-layer network");
   hipLaunchKernelGGL((dense_net<L, MT, TRAIN>), dim3((B + 16 * MT - 1) / (16 * MT)), dim3(kDenseThreads), 0, s, sh,
                      params, pack, x, B, y, tr);
   hipcheck(hipGetLastError(), "dense layers");
