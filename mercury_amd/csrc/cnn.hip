@@ -28,11 +28,13 @@
 // What the layer-by-layer form cost (a GEMM or column sum per launch, fp32
 // activations through memory, 64-wide tiles half empty at 32 channels): 35
 // launches and 812 us per training step of 256 genomes, 0.67 us per scored
-// genome.  As these kernels, on MI355X: 125 us of kernels per step
-// (conv_features 34, conv_wgrad 34, conv_backward 24, the head's two 15 and
+// genome.  As these kernels, on MI355X: 129 us of kernels per step
+// (conv_features 35, conv_wgrad 35, conv_backward 26, the head's two 15 and
 // 11, conv_update 6), 0.064 us per scored genome.  conv_features is bound by
-// the 36 900 tanh of a genome (VALU issue), the training kernels, one genome
-// per CU at this batch, by the latency of their chains.
+// the 36 900 tanh of a genome (VALU issue: 0.85 wave64 instructions per
+// CU-cycle, where plain FP32 chains reach 0.88-0.92; the matrix cores are busy
+// 27 % of the time), the training kernels, one genome per CU at this batch, by
+// the latency of their chains.
 #include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
 

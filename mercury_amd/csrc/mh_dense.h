@@ -3,14 +3,15 @@
 // gradients of every layer's output) without leaving the workgroup, and
 // dense_wgrad turns the operands it leaves into weight and bias gradients
 // (or straight into Adam's update).  For networks of up to kDenseMaxLayers
-// layers of at most kDenseMaxWidth units; wider ones run layer by layer with
-// the kernels of mh_nn_kernels.h.
+// layers of at most kDenseMaxWidth units; wider ones, and large batches of
+// narrow ones on device buffers, run layer by layer with the kernels of
+// mh_nn_kernels.h.
 //
 // What bounds them: launches and latency, not arithmetic.  A step of the
 // 64-256-256-1 network on 512 rows is 0.2 GFLOP; as 15 launches (a GEMM per
 // layer and direction, column sums, batch assembly, loss, Adam) it took
 // 82 us, each launch 3-11 us however little it did; as these two it takes
-// 15 + 8 us and 2-3 us of gaps (an epoch of 30011 rows 5.05 -> 1.83 ms).
+// 15 + 5.5 us and 2-3 us of gaps (an epoch of 30011 rows 5.05 -> 1.65 ms).
 // Inside dense_net a full layer costs 3000 cycles of tanh (8 waves, 8 values
 // a lane) and 2000 of reading 128 KB of weights through one CU's cache.
 //

@@ -287,9 +287,8 @@ __device__ __forceinline__ void mfma_tile(const LA& la, const LB& lb, int M, int
         put_slice<LB>(vb[s], sb[s]);
       }
     } else {
-      // one slice with checks: each operand written as soon as it is read
-      // (measured 10 % faster for the convolution weight gradients than
-      // reading both first)
+      // one slice with checks: each operand written as soon as it is read,
+      // which keeps one operand's values in registers instead of two
       put_slice<LA>(fetch_slice<true>(la, M, m0, k0, k_end), sa[0]);
       put_slice<LB>(fetch_slice<false>(lb, N, n0, k0, k_end), sb[0]);
     }

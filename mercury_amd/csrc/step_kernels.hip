@@ -1583,7 +1583,8 @@ __global__ void robot_com(const float4* pos, const uint8_t* mass_id, const uint3
 // step_mass for at most one workgroup per CU (force solver).  MI355X, us per
 // substep of the evaluate call, plain -> wide: one robot of 125 masses
 // (256-lane block, batches of 4) 3.4 -> 2.4, 256 of 343 masses (512) 4.8 ->
-// 3.8, one of 729 (768, batches of 2) 3.5 -> 3.2, 256 of them 5.5 -> 5.1.
+// 3.8; of a launch of 1000 substeps, 768 lanes and batches of 2: one of 125
+// masses 3.24 -> 2.21, one of 729 3.31 -> 2.76, 250 of them 3.37 -> 2.89.
 // 100 robots of 1000 masses (1024, batches of 2) went from 5.0 to 5.5: four
 // waves per SIMD cover the latency, so that block has none.
 template <int SOLVER, int B, int P>
